@@ -33,7 +33,7 @@ OP = {
     "CONST": 0, "LOAD": 1, "TIME": 2, "ADD": 3, "SUB": 4, "MUL": 5, "DIV": 6, "POW": 7,
     "POWI": 8, "NEG": 9, "STORE": 10, "SQRT": 11, "EXP": 12, "LOG": 13, "SIN": 14, "COS": 15,
     "TAN": 16, "TANH": 17, "ABS": 18, "ASIN": 19, "ACOS": 20, "ATAN": 21, "SINH": 22,
-    "COSH": 23, "ATAN2": 24, "MIN": 25, "MAX": 26, "SIGN": 27,
+    "COSH": 23, "ATAN2": 24, "MIN": 25, "MAX": 26, "SIGN": 27, "POW3H": 28,
 }
 MAX_REGS = 96  # PML_EXPR_MAX_REGS
 MAX_IO = 48  # PML_EXPR_MAX_IO
@@ -198,6 +198,8 @@ class _Builder:
                 return self.bin("DIV", one, self.un("SQRT", self.expr(base)))
             if ex.is_Number and float(ex).is_integer() and abs(float(ex)) < 2**31:
                 return self.un("POWI", self.expr(base), int(float(ex)))
+            if ex.is_Number and float(ex) == 1.5:
+                return self.un("POW3H", self.expr(base))
             return self.bin("POW", self.expr(base), self.expr(ex))
         for cls, op in _UNARY.items():
             if isinstance(e, cls):
@@ -303,7 +305,7 @@ def evaluate_on_host(program: Program, inputs: Sequence[np.ndarray], t: float) -
     fn = {"SQRT": np.sqrt, "EXP": np.exp, "LOG": np.log, "SIN": np.sin, "COS": np.cos,
           "TAN": np.tan, "TANH": np.tanh, "ABS": np.abs, "ASIN": np.arcsin, "ACOS": np.arccos,
           "ATAN": np.arctan, "SINH": np.sinh, "COSH": np.cosh, "NEG": np.negative,
-          "SIGN": np.sign}
+          "SIGN": np.sign, "POW3H": lambda x: np.power(x, 1.5)}
     with np.errstate(all="ignore"):
         for op, dst, a, b in program.code.tolist():
             name = inv[op]

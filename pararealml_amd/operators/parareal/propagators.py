@@ -21,7 +21,7 @@ slices at once:
 
 * ``ODESlicePropagator`` -- an ``FDMOperator`` on a system without a mesh:
   all requested slices advance together in one launch of the ODE kernel
-  (``pml_ode_solve``, one thread per slice, the whole slice in the launch),
+  (``pml_ode_solve``, the whole slice in the launch),
   each from its own start time.
 
 Every slice's initial value has the problem's static Dirichlet values
