@@ -87,6 +87,8 @@ extern "C" {
 /* Blocks of the fixed-order reductions (update and Jacobi norms): their
  * workspaces hold this many partial sums per reduced quantity. */
 #define PML_REDUCE_SLOTS 2048
+/* Stencil terms of pml_laplacian_solve at most. */
+#define PML_LAPLACIAN_MAX_TERMS 6
 /* Bytes of the state buffer of pml_jacobi_solve / pml_jacobi_solve_weighted. */
 #define PML_JACOBI_STATE_BYTES (32 + 8 * PML_REDUCE_SLOTS)
 
@@ -318,6 +320,31 @@ int pml_jacobi_solve_weighted(int precision, void *y, void *work, const void *la
                               void *state, int64_t *sweeps_out, double *diff_out,
                               const double *const *w_sum, const double *const *w_diff,
                               const double *w_den, void *stream);
+
+/*
+ * The whole explicit time loop of u_t = coefficient lap(u) on one grid of
+ * shape[0] x shape[1] x shape[2] vertices (C order, one field; unused
+ * trailing axes 1), where lap is the sum, in order, of n_terms stencils:
+ * term k is the first (term_order[k] = 1) or second (2) difference along
+ * axis term_axis[k] with the boundary rules of pml_stencil_first /
+ * pml_stencil_second (ghost_lo / ghost_hi: per-axis boundary arrays in the
+ * "axis removed" layout, NULL arrays or entries: none), times
+ * term_weight[k] (per-vertex, in the given precision; NULL array or entry:
+ * 1).  Covers Cartesian, polar, cylindrical and spherical meshes.  Every
+ * stage input and every step's result get the y constraints (ycons: FP64
+ * per vertex, NaN where free; NULL: none).  y holds the start and receives
+ * the end state; work holds 3 more states; snapshots (FP64) receives every
+ * snapshot_every-th state.  The stages round as the separate stencil,
+ * pml_weighted_add and pml_set_values calls do.  PML_F64 and PML_F32.
+ */
+int pml_laplacian_solve(int precision, int integrator_id, const int64_t *shape,
+                        const double *dx, const double *const *ghost_lo,
+                        const double *const *ghost_hi, int n_terms,
+                        const int *term_axis, const int *term_order,
+                        const void *const *term_weight, const double *ycons,
+                        double coefficient, double dt, int64_t n_steps, void *y,
+                        void *work, double *snapshots, int64_t snapshot_every,
+                        void *stream);
 
 /*
  * Parareal, all FP64.

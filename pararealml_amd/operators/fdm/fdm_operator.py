@@ -462,6 +462,16 @@ class FDMOperator(Operator):
             static = (encode(cp.static_y_vertex_constraints),
                       no_dbc(cp.static_boundary_vertex_constraints[1]),
                       cp.static_y_vertex_constraints)
+        if family == "diffusion" and not dynamic and not implicit and mesh.dimensions <= 3:
+            # the right-hand side is one Laplacian: fused stages, no host work
+            # between them
+            y = torch.from_numpy(np.ascontiguousarray(
+                ivp.initial_condition.discrete_y_0(True))).to(device="cuda", dtype=dtype)
+            dev_y = torch.empty((n_snap,) + shape, dtype=torch.float64, device="cuda")
+            diff.solve_laplacian(integ, mesh, y, dev_y, every, params[1][0], self._d_t, n_steps,
+                                 static[0], static[1])
+            return DeviceSolution(ivp, t[every::every], dev_y.cpu().numpy(), dev_y,
+                                  vertex_oriented=True, d_t=self._d_t * every)
         cache = {}
 
         def constraints_at(t_c):

@@ -507,28 +507,67 @@ class ThreePointCentralDifferenceMethod(NumericalDifferentiator):
         self._laplacian_terms(out, t, mesh, dbc)
         return out.out
 
+    @staticmethod
+    def laplacian_stencils(mesh: Mesh):
+        """The scalar Laplacian as a sum of stencils in the order they are
+        accumulated: (axis, order of the difference, per-vertex factor or
+        None)."""
+        cs = mesh.coordinate_system_type
+        if cs == CoordinateSystem.CARTESIAN:
+            return [(axis, 2, None) for axis in range(mesh.dimensions)]
+        r, sin_phi, cos_phi = _polar_factors(mesh)
+        if cs == CoordinateSystem.SPHERICAL:
+            return [(0, 2, None), (0, 1, 2.0 / r), (2, 2, 1.0 / (r * r)),
+                    (2, 1, cos_phi / (r * r * sin_phi)), (1, 2, 1.0 / (r * sin_phi) ** 2)]
+        terms = [(0, 2, None), (1, 2, 1.0 / (r * r)), (0, 1, 1.0 / r)]
+        if cs == CoordinateSystem.CYLINDRICAL:
+            terms.append((2, 2, None))
+        return terms
+
     def _laplacian_terms(self, out, t, mesh, dbc):
         for axis in range(t.dim() - 1):
             self._require_points(t.shape, axis)
-        d = mesh.d_x
-        cs = mesh.coordinate_system_type
-        if cs == CoordinateSystem.CARTESIAN:
-            for axis in range(t.dim() - 1):
-                out.second(t, axis, d[axis], dbc[axis, :])
-        elif cs == CoordinateSystem.SPHERICAL:
-            r, sin_phi, cos_phi = _polar_factors(mesh)
-            out.second(t, 0, d[0], dbc[0, :])
-            out.first(t, 0, d[0], dbc[0, :], 2.0 / r)
-            out.second(t, 2, d[2], dbc[2, :], 1.0 / (r * r))
-            out.first(t, 2, d[2], dbc[2, :], cos_phi / (r * r * sin_phi))
-            out.second(t, 1, d[1], dbc[1, :], 1.0 / (r * sin_phi) ** 2)
-        else:
-            r, _, _ = _polar_factors(mesh)
-            out.second(t, 0, d[0], dbc[0, :])
-            out.second(t, 1, d[1], dbc[1, :], 1.0 / (r * r))
-            out.first(t, 0, d[0], dbc[0, :], 1.0 / r)
-            if cs == CoordinateSystem.CYLINDRICAL:
-                out.second(t, 2, d[2], dbc[2, :])
+        for axis, order, coef in self.laplacian_stencils(mesh):
+            term = out.second if order == 2 else out.first
+            term(t, axis, mesh.d_x[axis], dbc[axis, :], coef)
+
+    def solve_laplacian(self, integrator: int, mesh: Mesh, y, snapshots, every: int,
+                        coefficient: float, d_t: float, n_steps: int, ycons,
+                        derivative_boundary_constraints) -> None:
+        """The explicit time loop of ``u_t = coefficient * laplacian(u)`` in
+        one call (``pml_laplacian_solve``): ``y`` (device, one field) holds
+        the start, ``snapshots`` (FP64) receives every ``every``-th state;
+        ``ycons`` are the y constraints as an FP64 device array, NaN where
+        free."""
+        import torch
+
+        a = _Arr(y)
+        shape = tuple(y.shape)
+        dims = mesh.dimensions
+        for axis in range(dims):
+            self._require_points(shape, axis)
+        spatial = list(shape[:-1]) + [1] * (3 - dims)
+        dxs = list(mesh.d_x) + [1.0] * (3 - dims)
+        keep, ghosts = [], ([], [])
+        for axis in range(3):
+            for side in (0, 1):
+                s = _slab_array(derivative_boundary_constraints[axis], side, shape, axis) \
+                    if axis < dims else None
+                keep.append(s)
+                ghosts[side].append(None if s is None else s.data_ptr())
+        terms = self.laplacian_stencils(mesh)
+        weights = [None if c is None else _weights(a, c, shape) for _, _, c in terms]
+        n = len(terms)
+        work = torch.empty((3,) + shape, dtype=a.t.dtype, device=a.t.device)
+        nat.check(nat.device_lib().pml_laplacian_solve(
+            a.prec, integrator, (ctypes.c_int64 * 3)(*spatial), (ctypes.c_double * 3)(*dxs),
+            (ctypes.c_void_p * 3)(*ghosts[0]), (ctypes.c_void_p * 3)(*ghosts[1]), n,
+            (ctypes.c_int * n)(*[axis for axis, _, _ in terms]),
+            (ctypes.c_int * n)(*[order for _, order, _ in terms]),
+            (ctypes.c_void_p * n)(*[None if w is None else w.data_ptr() for w in weights]),
+            None if ycons is None else ycons.data_ptr(), float(coefficient), float(d_t),
+            int(n_steps), a.t.data_ptr(), work.data_ptr(), snapshots.data_ptr(), int(every),
+            _stream()))
 
     def vector_laplacian(
         self, y, mesh: Mesh, vector_laplacian_ind: int, derivative_boundary_constraints=None
