@@ -287,7 +287,8 @@ int pml_jacobi_sweep(int precision, const void *y_old, void *y_new,
  * 872-927): sweeps (as pml_jacobi_sweep, y -> work -> y ...) until
  * ||y_new - y_old||_2 <= tol, with the stopping test on the device (a sweep
  * after convergence does nothing) and the host reading the loop state once
- * per `batch` sweeps.  y holds the start (constraints already applied) and
+ * per `batch` sweeps; a grid that fits one workgroup's memory runs the whole
+ * loop in one launch (the host looks once per 16384 sweeps).  y holds the start (constraints already applied) and
  * receives the result; work is a second array of the same size; state is a
  * device buffer of PML_JACOBI_STATE_BYTES (8-byte aligned).  The update
  * norm is summed in a fixed order, so the sweep count and the result are
@@ -345,6 +346,33 @@ int pml_laplacian_solve(int precision, int integrator_id, const int64_t *shape,
                         double coefficient, double dt, int64_t n_steps, void *y,
                         void *work, double *snapshots, int64_t snapshot_every,
                         void *stream);
+
+/*
+ * The time loop of an equation with LHS.Y_LAPLACIAN fields on one 2-D grid
+ * (fdm_operator.py:127-161): n_steps times one pml_fdm_solve step, after
+ * which each of the n_poisson fields is re-solved by Jacobi sweeps
+ * (pml_jacobi_solve) from lap(field[k]) = scale[k] * (pre-step source[k]),
+ * started from its pre-step value.  ghost_lo / ghost_hi hold 3 entries per
+ * field, ycons one (FP64 per vertex, NaN where free; NULL: none).  state
+ * holds the start and receives the end, work is a second state, snapshots
+ * (FP64, NULL: none) receives every snapshot_every-th state, jacobi_state is
+ * a device buffer of PML_JACOBI_STATE_BYTES.  *sweeps_out = the last solve's
+ * sweeps, or 0 where the grid is too large for the device loop (nothing was
+ * done) or a solve needs more than 16384 sweeps (state and snapshots are then
+ * unspecified) or there was no step: step with
+ * pml_fdm_solve and pml_jacobi_solve instead.  PML_F64 and PML_F32.
+ */
+int pml_fdm_poisson_solve(int eq_id, const double *eq_params, int n_params,
+                          int integrator_id, int precision, const pml_grid *grid,
+                          const double *bc_values, void *state, void *work,
+                          int64_t total_elems, double dt, int64_t n_steps,
+                          int tile_config, int n_poisson, const int *field,
+                          const int *source, const double *scale,
+                          const double *const *ghost_lo,
+                          const double *const *ghost_hi,
+                          const double *const *ycons, double tol,
+                          double *snapshots, int64_t snapshot_every,
+                          void *jacobi_state, int64_t *sweeps_out, void *stream);
 
 /*
  * Parareal, all FP64.

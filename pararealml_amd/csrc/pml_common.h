@@ -35,6 +35,12 @@ int fail(int code, const std::string &msg);
     }                                                                         \
   } while (0)
 
+// One step of pml_fdm_solve from `in` into `out` (whole states, FP32 or FP64),
+// without the copy back that a call of an odd number of steps ends with.
+int fdm_step(int eq_id, const double *eq_params, int n_params, int integrator_id, int precision,
+             int ndim, const pml_grid *grids, int n_grids, const double *bc_values, void *in,
+             void *out, int64_t total_elems, double dt, int tile_config, void *stream);
+
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
 // ---------------------------------------------------------------------------

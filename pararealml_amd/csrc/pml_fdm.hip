@@ -273,7 +273,7 @@ static int fdm_solve_impl(int eq_id, const double *eq_params, int n_params,
                           void *state_lo, void *work_hi, void *work_lo, int64_t total_elems,
                           double dt, int64_t n_steps, void *snapshots_hi,
                           void *snapshots_lo, int64_t snapshot_every, int tile_config,
-                          int flags, void *stream, bool no_alloc) {
+                          int flags, void *stream, bool no_alloc, bool leave = false) {
   int n_fields = 0;
   if (ndim != 1 && ndim != 2) return fail(PML_E_INVALID, "ndim must be 1 or 2");
   const auto *vars = find_variants(eq_id, integrator_id, precision, ndim, &n_fields);
@@ -515,13 +515,21 @@ static int fdm_solve_impl(int eq_id, const double *eq_params, int n_params,
     rc = launch(V.fn_single, 1);
     if (rc) return rc;
   }
-  if (cur_hi != state_hi) {
+  if (cur_hi != state_hi && !leave) {
     PML_HIP_CHECK(hipMemcpyAsync(state_hi, cur_hi, total_elems * esz, hipMemcpyDeviceToDevice, st));
     if (precision == PML_F32C)
       PML_HIP_CHECK(
           hipMemcpyAsync(state_lo, cur_lo, total_elems * esz, hipMemcpyDeviceToDevice, st));
   }
   return PML_OK;
+}
+
+int fdm_step(int eq_id, const double *eq_params, int n_params, int integrator_id, int precision,
+             int ndim, const pml_grid *grids, int n_grids, const double *bc_values, void *in,
+             void *out, int64_t total_elems, double dt, int tile_config, void *stream) {
+  return fdm_solve_impl(eq_id, eq_params, n_params, integrator_id, precision, ndim, grids,
+                        n_grids, bc_values, in, nullptr, out, nullptr, total_elems, dt, 1,
+                        nullptr, nullptr, 0, tile_config, 0, stream, false, true);
 }
 
 }  // namespace pml

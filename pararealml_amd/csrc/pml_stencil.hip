@@ -4,7 +4,10 @@
 // pararealml/operators/fdm/numerical_differentiator.py:1012-1242.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
+#include <type_traits>
+#include <vector>
 
 #include "pml_common.h"
 
@@ -195,6 +198,8 @@ struct JacobiGeom {
   const double *ghi[3];
   int active[3];
   double coef;  // sum over active axes of 2 / dx^2
+  // reciprocals of dxsq and coef, rounded in the precision of the sweep
+  double rdxsq[3], rcoef;
   // Curvilinear weights per vertex (NULL: Cartesian): the update is
   // (sum_a wsum[a] (prev + next) + wdiff[a] (next - prev) - lap) / wden.
   const double *wsum[3];
@@ -217,6 +222,67 @@ struct JacobiState {
 };
 static_assert(sizeof(JacobiState) == PML_JACOBI_STATE_BYTES, "JacobiState layout");
 
+// x / d with r = 1 / d rounded to nearest: the product with r, two steps of
+// correction by the residual x - q d (exact in one fused multiply-add).  The
+// first brings q within one ulp, after which the second rounds correctly
+// (P. Markstein, "Computation of elementary functions on the IBM RISC
+// System/6000 processor", 1990), so the result is the quotient's for every
+// normal x / d; 5 operations where the compiler's division takes 11 and a
+// reciprocal.
+template <typename T>
+__device__ __forceinline__ T div_by(T x, T d, T r) {
+  T q = x * r;
+  q = __builtin_elementwise_fma(__builtin_elementwise_fma(-d, q, x), r, q);
+  return __builtin_elementwise_fma(__builtin_elementwise_fma(-d, q, x), r, q);
+}
+
+// The update of element t (field f of cell (idx)) from the iterate y.
+template <typename T, typename I>
+__device__ __forceinline__ T jacobi_update(const T *y, I t, I f, I cell, const I *idx, I nf,
+                                           const JacobiGeom &g, T lap, const double *ycons) {
+  // constrained vertices, most often all of an edge's, need no neighbours
+  if (ycons) {
+    const double c = ycons[t];
+    if (c == c) return static_cast<T>(c);
+  }
+  T acc = 0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    if (!g.active[a]) continue;
+    const I s = static_cast<I>(g.stride[a]);
+    const I n = static_cast<I>(g.n[a]);
+    // Slab index: the element with axis a removed.
+    I slab = 0;
+    for (int b = 0; b < 3; ++b) {
+      if (b == a) continue;
+      slab = slab * static_cast<I>(g.n[b]) + idx[b];
+    }
+    slab = slab * nf + f;
+    T prev, next;
+    if (idx[a] > 0) {
+      prev = y[t - s];
+    } else {
+      const double gv = g.glo[a] ? g.glo[a][slab] : NAN;
+      prev = (gv == gv) ? y[t + s] + static_cast<T>(-2.0 * g.dx[a]) * static_cast<T>(gv) : T(0);
+    }
+    if (idx[a] < n - 1) {
+      next = y[t + s];
+    } else {
+      const double gv = g.ghi[a] ? g.ghi[a][slab] : NAN;
+      next = (gv == gv) ? y[t - s] + static_cast<T>(2.0 * g.dx[a]) * static_cast<T>(gv) : T(0);
+    }
+    if (g.wden) {
+      acc = acc + static_cast<T>(g.wsum[a][cell]) * (prev + next);
+      if (g.wdiff[a]) acc = acc + static_cast<T>(g.wdiff[a][cell]) * (next - prev);
+    } else {
+      acc = acc + div_by(prev + next, static_cast<T>(g.dxsq[a]), static_cast<T>(g.rdxsq[a]));
+    }
+  }
+  acc = acc - lap;
+  return g.wden ? acc / static_cast<T>(g.wden[cell])
+                : div_by(acc, static_cast<T>(g.coef), static_cast<T>(g.rcoef));
+}
+
 // Each block writes its sum of squared updates to partials[blockIdx.x]
 // (grid-stride order, then a fixed tree); k_jacobi_check adds them in block
 // order, so the norm and the sweep count do not depend on scheduling.
@@ -236,43 +302,7 @@ __global__ void k_jacobi(const T *y, T *yn, const T *lap, int64_t total, int nf,
     idx[2] = cell % g.n[2];
     idx[1] = (cell / g.n[2]) % g.n[1];
     idx[0] = cell / (g.n[2] * g.n[1]);
-    T acc = 0;
-    for (int a = 0; a < 3; ++a) {
-      if (!g.active[a]) continue;
-      const int64_t s = g.stride[a];
-      // Slab index: the element with axis a removed.
-      int64_t slab = 0;
-      for (int b = 0; b < 3; ++b) {
-        if (b == a) continue;
-        slab = slab * g.n[b] + idx[b];
-      }
-      slab = slab * nf + f;
-      T prev, next;
-      if (idx[a] > 0) {
-        prev = y[t - s];
-      } else {
-        const double gv = g.glo[a] ? g.glo[a][slab] : NAN;
-        prev = (gv == gv) ? y[t + s] + static_cast<T>(-2.0 * g.dx[a]) * static_cast<T>(gv) : T(0);
-      }
-      if (idx[a] < g.n[a] - 1) {
-        next = y[t + s];
-      } else {
-        const double gv = g.ghi[a] ? g.ghi[a][slab] : NAN;
-        next = (gv == gv) ? y[t - s] + static_cast<T>(2.0 * g.dx[a]) * static_cast<T>(gv) : T(0);
-      }
-      if (g.wden) {
-        acc = acc + static_cast<T>(g.wsum[a][cell]) * (prev + next);
-        if (g.wdiff[a]) acc = acc + static_cast<T>(g.wdiff[a][cell]) * (next - prev);
-      } else {
-        acc = acc + (prev + next) / static_cast<T>(g.dxsq[a]);
-      }
-    }
-    acc = acc - lap[t];
-    T v = acc / static_cast<T>(g.wden ? g.wden[cell] : g.coef);
-    if (ycons) {
-      const double c = ycons[t];
-      if (c == c) v = static_cast<T>(c);
-    }
+    const T v = jacobi_update<T, int64_t>(y, t, f, cell, idx, nf, g, lap[t], ycons);
     const double d = static_cast<double>(v) - static_cast<double>(y[t]);
     acc2 += d * d;
     yn[t] = v;
@@ -284,6 +314,179 @@ __global__ void k_jacobi(const T *y, T *yn, const T *lap, int64_t total, int nf,
     __syncthreads();
   }
   if (threadIdx.x == 0) partials[blockIdx.x] = red[0];
+}
+
+// The whole loop in one workgroup, the iterate in LDS: a sweep is two
+// barriers instead of two launches, and a caller that steps in time never
+// waits for the host to see the stopping test.  y (the iterate, overwritten
+// by the result) starts from `start`; the source is scale * lap.  Takes at
+// most `most` sweeps; a loop that has not reached tol by then leaves
+// state->done 0.  A state that holds an unfinished loop (state->pad set by an
+// earlier launch of the same time loop) makes the launch a no-op.
+//
+// One CU works on the grid.  A sweep is bound by the instructions of its
+// vertices (some 35 in 2-D, 16 wavefronts on 4 SIMDs) above 64 x 64 and by
+// its reduction and two barriers (1.2 us) below 20 x 20.
+// PLATE: one field on two axes, without vertex weights (grids of 3 x 3 and
+// more).  Vertices inside the grid read their neighbours without a branch
+// there; the general update is left to free vertices on an edge.
+template <typename T, int PER, bool PLATE>
+__global__ void __launch_bounds__(1024)
+    k_jacobi_resident(T *y, const T *start, const T *__restrict__ lap, T scale, int total, int nf,
+                      JacobiGeom g, const double *__restrict__ ycons, double tol, long long most,
+                      JacobiState *state) {
+  extern __shared__ unsigned char smem[];
+  double *part = reinterpret_cast<double *>(smem);  // one sum per wavefront
+  T *L = reinterpret_cast<T *>(smem + 16 * sizeof(double));
+  if (state->pad) return;  // the same value in every thread
+  const int tid = threadIdx.x, nt = blockDim.x;
+  // the source and which vertices are free stay in registers: a sweep reads
+  // nothing but the iterate (and boundary values where they are constrained)
+  T src[PER];
+  unsigned free = 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int t = tid + k * nt;
+    src[k] = T(0);
+    if (t < total) {
+      const double c = ycons ? ycons[t] : NAN;
+      L[t] = c == c ? static_cast<T>(c) : start[t];
+      src[k] = scale * lap[t];
+      if (c != c) free |= 1u << k;
+    }
+  }
+  __syncthreads();
+  const int n2 = static_cast<int>(g.n[2]), n1 = static_cast<int>(g.n[1]);
+  // Quotients by multiplication: with m = ceil(2^32 / d), t m / 2^32 exceeds
+  // t / d by less than t / 2^32, which cannot reach the next integer while
+  // t d < 2^32 (here both are below 2^16).
+  auto inverse = [](int d) { return d == 1 ? 0u : static_cast<unsigned>(0xffffffffu / d) + 1u; };
+  auto quotient = [](int t, unsigned m) {
+    return m ? static_cast<int>(__umulhi(static_cast<unsigned>(t), m)) : t;
+  };
+  const unsigned mf = inverse(nf), m2 = inverse(n2), m1 = inverse(n1);
+  const int n0 = static_cast<int>(g.n[0]);
+  const T dxsq0 = static_cast<T>(g.dxsq[0]), dxsq1 = static_cast<T>(g.dxsq[1]);
+  const T rdxsq0 = static_cast<T>(g.rdxsq[0]), rdxsq1 = static_cast<T>(g.rdxsq[1]);
+  const T coef = static_cast<T>(g.coef), rcoef = static_cast<T>(g.rcoef);
+  long long sweeps = 0;
+  double norm = 0.0, sum = 0.0;
+  bool done = false;
+  int stuck = 0;  // consecutive norms that are not a number
+  while (!done && sweeps < most && stuck < 3) {
+    T nv[PER];
+    double acc2 = 0.0;
+    int first = tid;
+    // Their indices are computed again in every sweep (kept, they are more
+    // than the registers hold).
+    if (PER > 2) asm volatile("" : "+v"(first));
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int t = first + k * nt;
+      if (free >> k & 1u) {
+        const T old = L[t];
+        int idx[3] = {0, 0, 0};
+        if (PLATE) {
+          const T up = L[max(t - n1, 0)], down = L[min(t + n1, total - 1)];
+          const T left = L[max(t - 1, 0)], right = L[min(t + 1, total - 1)];
+          idx[0] = quotient(t, m1);
+          idx[1] = t - idx[0] * n1;
+          T acc = T(0) + div_by(up + down, dxsq0, rdxsq0);
+          acc = acc + div_by(left + right, dxsq1, rdxsq1);
+          nv[k] = div_by(acc - src[k], coef, rcoef);
+          if (idx[0] == 0 || idx[0] == n0 - 1 || idx[1] == 0 || idx[1] == n1 - 1)
+            nv[k] = jacobi_update<T, int>(L, t, 0, t, idx, 1, g, src[k], nullptr);
+        } else {
+          const int cell = quotient(t, mf), f = t - cell * nf;
+          const int row = quotient(cell, m2);
+          idx[2] = cell - row * n2;
+          idx[0] = quotient(row, m1);
+          idx[1] = row - idx[0] * n1;
+          nv[k] = jacobi_update<T, int>(L, t, f, cell, idx, nf, g, src[k], nullptr);
+        }
+        const double d = static_cast<double>(nv[k]) - static_cast<double>(old);
+        acc2 += d * d;
+      }
+      if (PER > 2) __builtin_amdgcn_sched_barrier(0);
+    }
+    for (int s = 32; s > 0; s >>= 1) acc2 += __shfl_xor(acc2, s);
+    if ((tid & 63) == 0) part[tid >> 6] = acc2;
+    __syncthreads();  // every read of the iterate is done, the sums are there
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int t = tid + k * nt;
+      if (free >> k & 1u) L[t] = nv[k];
+    }
+    sum = 0.0;
+    for (int w = 0; w < nt >> 6; ++w) sum += part[w];
+    norm = sqrt(sum);
+    ++sweeps;
+    done = norm <= tol;
+    // A value that is not finite stays on its free neighbours for good (it
+    // is gone after one sweep where it has none): no later sweep can stop
+    // the loop, which its caller reports as not converging.
+    stuck = norm != norm ? stuck + 1 : 0;
+    __syncthreads();
+  }
+  for (int t = tid; t < total; t += nt) y[t] = L[t];
+  if (tid == 0) {
+    state->sumsq = sum;
+    state->last_diff = norm;
+    state->sweeps = sweeps;
+    state->done = done ? 1 : (stuck >= 3 ? -1 : 0);
+    if (!done) state->pad = 1;
+  }
+}
+
+// Whether the resident loop takes a grid, and its workgroup memory.  A sweep
+// of two launches takes 8 to 9 us whatever the size (of these), and 64 are
+// launched before the host looks.  Resident sweeps in FP64: plates between
+// constrained edges 1.2 us at 17 x 17, 2.7 at 64 x 64, 5.6 at 100 x 100, 8.0
+// at 129 x 129; with free edges (the general update in every wavefront) 2.3
+// at 45 x 45, 4.8 at 64 x 64, 9.4 at 100 x 100; other grids
+// 2.0 at 13^3, 5.4 at 17^3.  The lid-driven cavity on 65 x 65, 60 steps: 42 ms
+// with a host round trip and 128 launches a step, 1.6 ms in the device loop.
+constexpr int kResidentPer = 18;
+// Sweeps of one launch at most (some 100 ms on the largest grid): the host
+// looks at the loop's state in between.
+constexpr int64_t kResidentSweeps = 16384;
+template <typename T>
+static size_t resident_lds(int64_t total) {
+  return 16 * sizeof(double) + sizeof(T) * static_cast<size_t>(total);
+}
+static bool is_plate(const JacobiGeom &g, int nf) {
+  return nf == 1 && !g.wden && g.n[0] > 1 && g.n[1] > 1 && g.n[2] == 1;
+}
+static bool takes_resident(int precision, int64_t total, int nf, const JacobiGeom &g,
+                           bool constrained) {
+  const size_t lds = precision == PML_F64 ? resident_lds<double>(total) : resident_lds<float>(total);
+  const int64_t limit = !is_plate(g, nf) ? 5 * 1024 : (constrained ? kResidentPer * 1024 : 8 * 1024);
+  return total <= limit && lds <= 150 * 1024;
+}
+
+template <typename T>
+static int launch_resident(T *y, const T *start, const T *lap, T scale, int64_t total, int nf,
+                           const JacobiGeom &g, const double *ycons, double tol, long long most,
+                           JacobiState *state, hipStream_t st) {
+  const size_t lds = resident_lds<T>(total);
+  const int threads = total < 1024 ? static_cast<int>((total + 63) / 64 * 64) : 1024;
+  auto launch = [&](auto kernel) -> int {
+    PML_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), lds, st, y, start, lap, scale,
+                       static_cast<int>(total), nf, g, ycons, tol, most, state);
+    PML_LAUNCH_CHECK();
+    return PML_OK;
+  };
+  const bool plate = is_plate(g, nf);
+  auto pick = [&](auto per) {
+    constexpr int P = decltype(per)::value;
+    return plate ? launch(&k_jacobi_resident<T, P, true>)
+                 : launch(&k_jacobi_resident<T, P, false>);
+  };
+  if (total <= 2 * 1024) return pick(std::integral_constant<int, 2>{});
+  if (total <= 5 * 1024) return pick(std::integral_constant<int, 5>{});
+  return pick(std::integral_constant<int, kResidentPer>{});
 }
 
 // sum of parts[0 .. n) in a fixed order into *out (one block).
@@ -587,7 +790,7 @@ extern "C" int pml_laplacian_solve(int precision, int integrator_id, const int64
 
 // Geometry of a Jacobi sweep over a (shape[0], shape[1], shape[2], n_fields)
 // array; returns PML_OK or the error, and the element count in *total.
-static int jacobi_geom(const int64_t *shape, int n_fields, const double *dx,
+static int jacobi_geom(int precision, const int64_t *shape, int n_fields, const double *dx,
                        const double *const *ghost_lo, const double *const *ghost_hi,
                        JacobiGeom *out, int64_t *total_out) {
   JacobiGeom g{};
@@ -607,8 +810,13 @@ static int jacobi_geom(const int64_t *shape, int n_fields, const double *dx,
       if (!(dx[a] > 0)) return fail(PML_E_INVALID, "spacing must be positive");
       g.coef += 2.0 / g.dxsq[a];
     }
+    g.rdxsq[a] = precision == PML_F32
+                     ? static_cast<double>(1.0f / static_cast<float>(g.dxsq[a]))
+                     : 1.0 / g.dxsq[a];
     total *= shape[a];
   }
+  g.rcoef = precision == PML_F32 ? static_cast<double>(1.0f / static_cast<float>(g.coef))
+                                 : 1.0 / g.coef;
   g.stride[2] = n_fields;
   g.stride[1] = shape[2] * n_fields;
   g.stride[0] = shape[1] * shape[2] * n_fields;
@@ -626,7 +834,7 @@ extern "C" int pml_jacobi_sweep(int precision, const void *y_old, void *y_new, c
     return fail(PML_E_INVALID, "bad Jacobi arguments");
   JacobiGeom g{};
   int64_t total = 0;
-  if (int rc = jacobi_geom(shape, n_fields, dx, ghost_lo, ghost_hi, &g, &total); rc != PML_OK)
+  if (int rc = jacobi_geom(precision, shape, n_fields, dx, ghost_lo, ghost_hi, &g, &total); rc != PML_OK)
     return rc;
   hipStream_t st = as_stream(stream);
   int nb = grid_for(total);
@@ -661,7 +869,7 @@ static int jacobi_solve(int precision, void *y, void *work, const void *lap,
     return fail(PML_E_INVALID, "Jacobi solve takes FP32 or FP64 arrays");
   JacobiGeom g{};
   int64_t total = 0;
-  if (int rc = jacobi_geom(shape, n_fields, dx, ghost_lo, ghost_hi, &g, &total); rc != PML_OK)
+  if (int rc = jacobi_geom(precision, shape, n_fields, dx, ghost_lo, ghost_hi, &g, &total); rc != PML_OK)
     return rc;
   if (w_den) {
     if (!w_sum) return fail(PML_E_INVALID, "weighted Jacobi needs w_sum");
@@ -677,12 +885,35 @@ static int jacobi_solve(int precision, void *y, void *work, const void *lap,
   JacobiState *js = static_cast<JacobiState *>(state);
   int nb = grid_for(total);
   if (nb > PML_REDUCE_SLOTS) nb = PML_REDUCE_SLOTS;
-  hipLaunchKernelGGL(k_jacobi_init, dim3(1), dim3(64), 0, st, js);
   JacobiState host;
   host.done = 0;
   host.sweeps = 0;
   host.last_diff = 0.0;
   int64_t issued = 0;
+  if (takes_resident(precision, total, n_fields, g, ycons != nullptr)) {
+    while (issued < max_sweeps) {
+      const int64_t n = std::min<int64_t>(kResidentSweeps, max_sweeps - issued);
+      hipLaunchKernelGGL(k_jacobi_init, dim3(1), dim3(64), 0, st, js);
+      const int rc =
+          precision == PML_F64
+              ? launch_resident<double>(static_cast<double *>(y), static_cast<const double *>(y),
+                                        static_cast<const double *>(lap), 1.0, total, n_fields, g,
+                                        ycons, tol, n, js, st)
+              : launch_resident<float>(static_cast<float *>(y), static_cast<const float *>(y),
+                                       static_cast<const float *>(lap), 1.0f, total, n_fields, g,
+                                       ycons, tol, n, js, st);
+      if (rc) return rc;
+      PML_HIP_CHECK(hipMemcpyAsync(&host, js, offsetof(JacobiState, partials),
+                                   hipMemcpyDeviceToHost, st));
+      PML_HIP_CHECK(hipStreamSynchronize(st));
+      issued = host.done < 0 ? max_sweeps : issued + host.sweeps;
+      if (host.done == 1) break;
+    }
+    *sweeps_out = host.done == 1 ? issued : -issued;
+    if (diff_out) *diff_out = host.last_diff;
+    return PML_OK;
+  }
+  hipLaunchKernelGGL(k_jacobi_init, dim3(1), dim3(64), 0, st, js);
   while (issued < max_sweeps) {
     const int64_t n = std::min<int64_t>(batch, max_sweeps - issued);
     for (int64_t k = 0; k < n; ++k) {
@@ -745,4 +976,86 @@ extern "C" int pml_jacobi_solve_weighted(int precision, void *y, void *work, con
   return jacobi_solve(precision, y, work, lap, shape, n_fields, dx, ghost_lo, ghost_hi, ycons,
                       tol, max_sweeps, batch, state, sweeps_out, diff_out, w_sum, w_diff, w_den,
                       stream);
+}
+
+extern "C" int pml_fdm_poisson_solve(int eq_id, const double *eq_params, int n_params,
+                                     int integrator_id, int precision, const pml_grid *grid,
+                                     const double *bc_values, void *state, void *work,
+                                     int64_t total_elems, double dt, int64_t n_steps,
+                                     int tile_config, int n_poisson, const int *field,
+                                     const int *source, const double *scale,
+                                     const double *const *ghost_lo,
+                                     const double *const *ghost_hi, const double *const *ycons,
+                                     double tol, double *snapshots, int64_t snapshot_every,
+                                     void *jacobi_state, int64_t *sweeps_out, void *stream) {
+  if (!grid || !state || !work || !field || !source || !scale || !ghost_lo || !ghost_hi ||
+      !ycons || !jacobi_state || !sweeps_out || n_poisson <= 0 || n_steps < 0 || !(tol >= 0.0) ||
+      (snapshots && snapshot_every <= 0))
+    return fail(PML_E_INVALID, "bad Poisson time loop arguments");
+  if (precision != PML_F64 && precision != PML_F32)
+    return fail(PML_E_UNSUPPORTED, "LHS.Y_LAPLACIAN equations run in FP32 or FP64");
+  *sweeps_out = 0;
+  const int64_t plane = static_cast<int64_t>(grid->n0) * grid->n1;
+  const int64_t shape[3] = {grid->n0, grid->n1, 1};
+  const double dx[3] = {grid->dx0, grid->dx1, 1.0};
+  if (plane <= 0 || plane > total_elems || grid->state_offset != 0)
+    return fail(PML_E_INVALID, "bad grid of a Poisson time loop");
+  const int64_t fields = total_elems / plane;
+  std::vector<JacobiGeom> geoms(n_poisson);
+  for (int k = 0; k < n_poisson; ++k) {
+    if (field[k] < 0 || field[k] >= fields || source[k] < 0 || source[k] >= fields)
+      return fail(PML_E_INVALID, "bad field of a Poisson equation");
+    int64_t total = 0;
+    if (int rc = jacobi_geom(precision, shape, 1, dx, ghost_lo + 3 * k, ghost_hi + 3 * k, &geoms[k],
+                             &total);
+        rc != PML_OK)
+      return rc;
+    if (!takes_resident(precision, plane, 1, geoms[k], ycons[k] != nullptr)) return PML_OK;
+  }
+  hipStream_t st = as_stream(stream);
+  auto *js = static_cast<JacobiState *>(jacobi_state);
+  const size_t esz = precision == PML_F64 ? 8 : 4;
+  hipLaunchKernelGGL(k_jacobi_init, dim3(1), dim3(64), 0, st, js);
+  PML_LAUNCH_CHECK();
+  char *cur = static_cast<char *>(state), *nxt = static_cast<char *>(work);
+  for (int64_t s = 0; s < n_steps; ++s) {
+    if (int rc = fdm_step(eq_id, eq_params, n_params, integrator_id, precision, 2, grid, 1,
+                          bc_values, cur, nxt, total_elems, dt, tile_config, stream);
+        rc != PML_OK)
+      return rc;
+    for (int k = 0; k < n_poisson; ++k) {
+      // the pre-step state's source, the iteration started from its field
+      const size_t f = static_cast<size_t>(field[k]) * plane * esz;
+      const size_t q = static_cast<size_t>(source[k]) * plane * esz;
+      const int rc =
+          precision == PML_F64
+              ? launch_resident<double>(reinterpret_cast<double *>(nxt + f),
+                                        reinterpret_cast<const double *>(cur + f),
+                                        reinterpret_cast<const double *>(cur + q), scale[k],
+                                        plane, 1, geoms[k], ycons[k], tol, kResidentSweeps, js,
+                                        st)
+              : launch_resident<float>(reinterpret_cast<float *>(nxt + f),
+                                       reinterpret_cast<const float *>(cur + f),
+                                       reinterpret_cast<const float *>(cur + q),
+                                       static_cast<float>(scale[k]), plane, 1, geoms[k],
+                                       ycons[k], tol, kResidentSweeps, js, st);
+      if (rc) return rc;
+    }
+    std::swap(cur, nxt);
+    if (snapshots && (s + 1) % snapshot_every == 0)
+      if (int rc = pml_to_f64(precision, cur, nullptr,
+                              snapshots + ((s + 1) / snapshot_every - 1) * total_elems,
+                              total_elems, stream);
+          rc != PML_OK)
+        return rc;
+  }
+  if (cur != state)
+    PML_HIP_CHECK(
+        hipMemcpyAsync(state, cur, total_elems * esz, hipMemcpyDeviceToDevice, st));
+  JacobiState host;
+  PML_HIP_CHECK(hipMemcpyAsync(&host, js, offsetof(JacobiState, partials), hipMemcpyDeviceToHost,
+                               st));
+  PML_HIP_CHECK(hipStreamSynchronize(st));
+  *sweeps_out = host.pad ? 0 : host.sweeps;
+  return PML_OK;
 }

@@ -850,6 +850,53 @@ class FDMOperator(Operator):
         return DeviceSolution(ivp, t[every::every], out, dev_y, vertex_oriented=True,
                               d_t=dt * every)
 
+    def _poisson_loop(self, batch, problem, y_cons, d_cons, tile, n_steps, traj, every) -> bool:
+        """The whole time loop on the device (``pml_fdm_poisson_solve``);
+        False where it does not cover the run, which then has to be stepped
+        from its initial state."""
+        import ctypes
+
+        import torch
+
+        from pararealml_amd.operators.fdm.numerical_differentiator import _slab_array
+
+        diff = self._differentiator
+        if diff._max_sweeps < 16384:  # the limit is the caller's own
+            return False
+        shape = (problem.n0, problem.n1, 1)
+        n = len(problem.y_laplacian)
+        ghosts, fixed = ([], []), []
+        for f, _, _ in problem.y_laplacian:
+            for axis in range(3):
+                for side in (0, 1):
+                    ghosts[side].append(
+                        None if d_cons is None or axis == 2
+                        else _slab_array(d_cons[axis, f:f + 1], side, shape, axis))
+            c = None if y_cons is None else y_cons[f]
+            if c is not None:
+                full = np.full(shape, np.nan)
+                full[c.mask] = c.values
+                c = torch.from_numpy(full.ravel()).to("cuda")
+            fixed.append(c)
+        jacobi = torch.empty(nat.PML_JACOBI_STATE_BYTES // 8, dtype=torch.float64, device="cuda")
+        sweeps = ctypes.c_int64(0)
+        pointers = lambda ts: (ctypes.c_void_p * len(ts))(  # noqa: E731
+            *[None if a is None else a.data_ptr() for a in ts])
+        nat.check(batch.lib.pml_fdm_poisson_solve(
+            batch.eq_id, batch._params, len(batch.params), batch.integrator, batch.prec,
+            ctypes.byref(batch.grids[0]), batch.bc.data_ptr(), batch.hi.data_ptr(),
+            batch.work_hi.data_ptr(), batch.total, float(self._d_t), int(n_steps), int(tile), n,
+            (ctypes.c_int * n)(*[f for f, _, _ in problem.y_laplacian]),
+            (ctypes.c_int * n)(*[src for _, src, _ in problem.y_laplacian]),
+            (ctypes.c_double * n)(*[c for _, _, c in problem.y_laplacian]),
+            pointers(ghosts[0]), pointers(ghosts[1]), pointers(fixed), float(diff._tol),
+            traj.data_ptr(), int(every), jacobi.data_ptr(), ctypes.byref(sweeps),
+            batch._sptr()))
+        if not sweeps.value:
+            return False
+        diff.last_jacobi_sweeps = int(sweeps.value)
+        return True
+
     def _solve_with_poisson(self, ivp, problem, integ, t, n_steps, every, y0) -> Solution:
         """The time loop for equations with LHS.Y_LAPLACIAN components
         (fdm_operator.py:141-161): each step runs the fused kernel (the
@@ -883,7 +930,10 @@ class FDMOperator(Operator):
             traj = torch.empty((n_snap, problem.elems), dtype=torch.float64, device="cuda")
             tile = self.tile_config_for(problem)
             state = batch.hi  # field-major, the batch precision
-            for i in range(n_steps):
+            fused = self._poisson_loop(batch, problem, y_cons, d_cons, tile, n_steps, traj, every)
+            if not fused:  # a large grid, or a solve of many sweeps
+                batch.load_host([y0])
+            for i in range(0 if fused else n_steps):
                 sources = {
                     f: (c * state[src * plane:(src + 1) * plane]).view(shape)
                     for f, src, c in problem.y_laplacian
