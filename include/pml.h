@@ -375,6 +375,23 @@ int pml_fdm_poisson_solve(int eq_id, const double *eq_params, int n_params,
                           void *jacobi_state, int64_t *sweeps_out, void *stream);
 
 /*
+ * Results for the host.
+ *   pml_channel_last: n_states field-major states (n_fields planes of `plane`
+ *     FP64 values, 1 to 4 fields) -> channel-last copies.
+ *   pml_download: copies `bytes` bytes from the device into ordinary host
+ *     memory after the work queued on the stream, and returns when they are
+ *     there.  Several host threads fill dst from pinned staging memory (at
+ *     most 2 x 16 MiB are kept between calls; pml_graph_cache_clear gives
+ *     them back).  Not for capture.
+ *   pml_host_copy: host memory to host memory (not overlapping), by as many
+ *     threads.
+ */
+int pml_channel_last(const double *field_major, double *channel_last,
+                     int n_fields, int64_t plane, int64_t n_states, void *stream);
+int pml_download(void *dst, const void *src, int64_t bytes, void *stream);
+int pml_host_copy(void *dst, const void *src, int64_t bytes);
+
+/*
  * Parareal, all FP64.
  *   pml_parareal_correction: corr[s] = f_end[s] - g_end[s] over n elements
  *     per slice, for slices [s0, s1).  f_end may be FP32 or compensated FP32

@@ -149,6 +149,54 @@ def device_problem(cp) -> DeviceProblem:
                          tuple(diff_eq.device_y_laplacian()))
 
 
+_THREADED_BYTES = 4 << 20
+
+
+def host_copy(a: np.ndarray) -> np.ndarray:
+    """A copy of a contiguous host array, by several threads where the first
+    touch of its pages would take one thread milliseconds."""
+    if a.nbytes < _THREADED_BYTES or not a.flags.c_contiguous:
+        return np.copy(a)
+    out = np.empty_like(a)
+    nat.check(nat.load_library().pml_host_copy(out.ctypes.data, a.ctypes.data, a.nbytes))
+    return out
+
+
+def to_host(t) -> np.ndarray:
+    """A contiguous device tensor as a NumPy array in ordinary memory, after
+    the work queued on the current stream.  Most of torch's copy is the first
+    touch of the destination's pages by one thread, which ``pml_download``
+    shares out: 82 MB 19.5 ms / 2.9 ms, 20 MB 3.6 / 0.8, 4 MB 0.24 / 0.23;
+    below that torch's copy has less to set up (2 MB 0.13 / 0.19)."""
+    import torch
+
+    nbytes = t.numel() * t.element_size()
+    if nbytes < _THREADED_BYTES or t.dtype not in (torch.float64, torch.float32):
+        return t.cpu().numpy()
+    out = np.empty(tuple(t.shape), dtype=np.float64 if t.dtype == torch.float64 else np.float32)
+    nat.check(nat.device_lib().pml_download(
+        out.ctypes.data, t.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream))
+    return out
+
+
+def states_to_host(states, problem, spatial_shape) -> np.ndarray:
+    """FP64 field-major device states ``(n, elems)`` of ``problem`` as a
+    channel-last host array ``(n, *spatial_shape, fields)``."""
+    import torch
+
+    n = states.shape[0]
+    if problem.n_fields > 1 and problem.plane > 1:
+        if 8 * states.numel() < 1 << 20:  # sooner transposed here than launched there
+            flat = states.cpu().numpy().reshape(n, problem.n_fields, problem.n0, problem.n1)
+            return problem.from_device_layout(flat, spatial_shape)
+        last = torch.empty_like(states)
+        nat.check(nat.device_lib().pml_channel_last(
+            states.data_ptr(), last.data_ptr(), problem.n_fields, problem.plane, n,
+            torch.cuda.current_stream().cuda_stream))
+        states = last
+    return to_host(states).reshape((n,) + tuple(spatial_shape) + (problem.n_fields,))
+
+
 _streams = {}
 
 

@@ -175,6 +175,11 @@ SIGNATURES = {
          POINTER(c_double), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), c_double,
          c_void_p, c_int64, c_void_p, POINTER(c_int64), c_void_p],
     ),
+    "pml_channel_last": (
+        c_int, [c_void_p, c_void_p, c_int, c_int64, c_int64, c_void_p]
+    ),
+    "pml_host_copy": (c_int, [c_void_p, c_void_p, c_int64]),
+    "pml_download": (c_int, [c_void_p, c_void_p, c_int64, c_void_p]),
     "pml_parareal_correction": (
         c_int,
         [c_int, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int64,

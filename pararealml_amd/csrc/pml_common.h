@@ -35,6 +35,9 @@ int fail(int code, const std::string &msg);
     }                                                                         \
   } while (0)
 
+// Frees the pinned staging memory that pml_download keeps between calls.
+void release_staging();
+
 // One step of pml_fdm_solve from `in` into `out` (whole states, FP32 or FP64),
 // without the copy back that a call of an odd number of steps ends with.
 int fdm_step(int eq_id, const double *eq_params, int n_params, int integrator_id, int precision,

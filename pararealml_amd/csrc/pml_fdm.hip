@@ -121,6 +121,7 @@ extern "C" int pml_graph_cache_clear(void) {
     if (kv.second.grids) hipFree(kv.second.grids);
   }
   g_tables.clear();
+  release_staging();
   return PML_OK;
 }
 

@@ -299,10 +299,8 @@ class FDMOperator(Operator):
                 use_graph=self._use_graph,
             )
             dev_y = batch.snapshots_f64(snaps, n_snap)
-            flat = dev_y.cpu().numpy()
+            y = dev.states_to_host(dev_y, problem, cp.mesh.vertices_shape)
         torch.cuda.current_stream().wait_stream(stream)
-        flat = flat.reshape(n_snap, problem.n_fields, problem.n0, problem.n1)
-        y = problem.from_device_layout(flat, cp.mesh.vertices_shape)
         return DeviceSolution(
             ivp,
             t[every::every],
@@ -311,6 +309,7 @@ class FDMOperator(Operator):
             vertex_oriented=True,
             d_t=self._d_t * every,
             field_major=True,
+            copy=False,
         )
 
     def _ode_precision(self) -> int:
@@ -373,10 +372,10 @@ class FDMOperator(Operator):
                                         y.data_ptr(), snaps.data_ptr(), int(every),
                                         stream.cuda_stream))
             dev_y = snaps.view(n_snap, n).to(torch.float64)
-            out = dev_y.cpu().numpy()
+            out = dev.to_host(dev_y)
         torch.cuda.current_stream().wait_stream(stream)
         return DeviceSolution(ivp, t[every::every], out, dev_y, vertex_oriented=True,
-                              d_t=self._d_t * every)
+                              d_t=self._d_t * every, copy=False)
 
     def _solve_composed(self, ivp: InitialValueProblem) -> Solution:
         """Polar, cylindrical and spherical meshes, 3-D Cartesian ones and
@@ -470,8 +469,8 @@ class FDMOperator(Operator):
             dev_y = torch.empty((n_snap,) + shape, dtype=torch.float64, device="cuda")
             diff.solve_laplacian(integ, mesh, y, dev_y, every, params[1][0], self._d_t, n_steps,
                                  static[0], static[1])
-            return DeviceSolution(ivp, t[every::every], dev_y.cpu().numpy(), dev_y,
-                                  vertex_oriented=True, d_t=self._d_t * every)
+            return DeviceSolution(ivp, t[every::every], dev.to_host(dev_y), dev_y,
+                                  vertex_oriented=True, d_t=self._d_t * every, copy=False)
         cache = {}
 
         def constraints_at(t_c):
@@ -846,9 +845,9 @@ class FDMOperator(Operator):
             if (step + 1) % every == 0:
                 snaps.append(y.clone())
         dev_y = torch.stack(snaps).to(torch.float64)
-        out = dev_y.cpu().numpy()
+        out = dev.to_host(dev_y)
         return DeviceSolution(ivp, t[every::every], out, dev_y, vertex_oriented=True,
-                              d_t=dt * every)
+                              d_t=dt * every, copy=False)
 
     def _poisson_loop(self, batch, problem, y_cons, d_cons, tile, n_steps, traj, every) -> bool:
         """The whole time loop on the device (``pml_fdm_poisson_solve``);
@@ -950,9 +949,7 @@ class FDMOperator(Operator):
                     cur.copy_(new)
                 if (i + 1) % every == 0:
                     batch.state_f64(traj[(i + 1) // every - 1])
-            flat = traj.cpu().numpy()
+            y = dev.states_to_host(traj, problem, mesh.vertices_shape)
         torch.cuda.current_stream().wait_stream(stream)
-        flat = flat.reshape(n_snap, problem.n_fields, problem.n0, problem.n1)
-        y = problem.from_device_layout(flat, mesh.vertices_shape)
         return DeviceSolution(ivp, t[every::every], y, traj, vertex_oriented=True,
-                              d_t=self._d_t * every, field_major=True)
+                              d_t=self._d_t * every, field_major=True, copy=False)

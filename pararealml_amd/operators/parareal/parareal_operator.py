@@ -278,21 +278,14 @@ class PararealOperator(Operator):
             self.last_iterations = iterations
             if self._output == "endpoints":
                 dev_y = f_end + (u[1:] - f_end)
-                shifted = dev_y.cpu().numpy()
-                y = problem.from_device_layout(
-                    shifted.reshape(n, n_fields, problem.n0, problem.n1),
-                    spatial,
-                )
+                y = dev.states_to_host(dev_y, problem, spatial)
                 t = borders[1:]
                 d_t_out = delta
             else:
                 traj = fine.trajectory_f64()  # (steps, n, elems)
                 shift = (u[1:] - traj[-1]).unsqueeze(0)
                 dev_y = (traj + shift).permute(1, 0, 2).reshape(n * f_steps, elems)
-                y = problem.from_device_layout(
-                    dev_y.cpu().numpy().reshape(n * f_steps, n_fields, problem.n0, problem.n1),
-                    spatial,
-                )
+                y = dev.states_to_host(dev_y, problem, spatial)
                 t = discretize_time_domain(ivp.t_interval, f.d_t)[1:]
                 d_t_out = f.d_t
         torch.cuda.current_stream().wait_stream(stream)
@@ -300,7 +293,7 @@ class PararealOperator(Operator):
             timings, iterations=iterations, update_norms=norms_hist, iteration_wall_s=iter_wall
         )
         return DeviceSolution(ivp, t, y, dev_y, vertex_oriented=self._vertex_oriented,
-                              d_t=d_t_out, field_major=True)
+                              d_t=d_t_out, field_major=True, copy=False)
 
 
 _LINEAR_FAMILIES = ("diffusion", "convection_diffusion", "wave")

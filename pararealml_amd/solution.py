@@ -27,6 +27,8 @@ class Solution:
         discrete_y: np.ndarray,
         vertex_oriented: Optional[bool] = None,
         d_t: Optional[float] = None,
+        *,
+        copy: bool = True,
     ):
         if t_coordinates.ndim != 1:
             raise ValueError(
@@ -48,7 +50,8 @@ class Solution:
             )
         self._ivp = ivp
         self._t_coordinates = np.array(t_coordinates, copy=True)
-        self._discrete_y = np.array(discrete_y, copy=True)
+        # copy=False: the caller hands over an array that nobody else holds
+        self._discrete_y = np.array(discrete_y, copy=True) if copy else discrete_y
         self._vertex_oriented = vertex_oriented
         self._t_coordinates.setflags(write=False)
         if d_t is None:
@@ -83,7 +86,7 @@ class Solution:
         cp = self._ivp.constrained_problem
         diff_eq = cp.differential_equation
         if not diff_eq.x_dimension:
-            return np.copy(self._discrete_y)
+            return self._values_copy()
         values = interpn(
             cp.mesh.axis_coordinates(self._vertex_oriented),
             np.moveaxis(self._discrete_y, 0, -2),
@@ -97,6 +100,9 @@ class Solution:
             (len(self._t_coordinates),) + x.shape[:-1] + (diff_eq.y_dimension,)
         )
         return np.ascontiguousarray(values)
+
+    def _values_copy(self) -> np.ndarray:
+        return np.copy(self._discrete_y)
 
     def discrete_y(
         self,
@@ -112,7 +118,7 @@ class Solution:
             not cp.differential_equation.x_dimension
             or self._vertex_oriented == vertex_oriented
         ):
-            return np.copy(self._discrete_y)
+            return self._values_copy()
         x = cp.mesh.all_index_coordinates(vertex_oriented)
         values = self.y(x, interpolation_method)
         if vertex_oriented:
@@ -194,8 +200,10 @@ class DeviceSolution(Solution):
         vertex_oriented: Optional[bool] = None,
         d_t: Optional[float] = None,
         field_major: bool = False,
+        *,
+        copy: bool = True,
     ):
-        super().__init__(ivp, t_coordinates, discrete_y, vertex_oriented, d_t)
+        super().__init__(ivp, t_coordinates, discrete_y, vertex_oriented, d_t, copy=copy)
         import torch
 
         if not isinstance(device_y, torch.Tensor) or not device_y.is_cuda:
@@ -211,6 +219,11 @@ class DeviceSolution(Solution):
         )
         self._coords = None
         self._time_inner = None
+
+    def _values_copy(self) -> np.ndarray:
+        from pararealml_amd import _device as dev
+
+        return dev.host_copy(self._discrete_y)
 
     @property
     def device_y(self):
@@ -318,7 +331,7 @@ class DeviceSolution(Solution):
         """Values at arbitrary spatial points for every time step
         (pararealml/solution.py:114-145), interpolated on the device."""
         if not self._ivp.constrained_problem.differential_equation.x_dimension:
-            return np.copy(self._discrete_y)
+            return self._values_copy()
         return np.ascontiguousarray(self.y_device(x, interpolation_method).cpu().numpy())
 
     def _device_stack(self, other: Solution):
