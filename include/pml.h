@@ -161,7 +161,12 @@ int pml_device_sync(void *stream);
  *                       (what the reference's initial conditions do);
  *                       PML_FLAG_PREPARE -- build (and cache) the unit
  *                       tables and the step-loop graph this call would use,
- *                       and launch nothing
+ *                       and launch nothing;
+ *                       PML_FLAG_AUTO -- run a batch of up to some 400000
+ *                       vertices by the many-step kernel (a tile and its
+ *                       halo per workgroup, several steps a launch, the
+ *                       snapshots of all of them) instead of tile_config,
+ *                       which larger batches keep; the results are the same
  * After the call the current state is in state_hi/lo.
  *
  * Work-unit tables are built once per distinct grid array and kept (device
@@ -174,6 +179,7 @@ int pml_device_sync(void *stream);
 #define PML_FLAG_GRAPH 1
 #define PML_FLAG_CONSTRAIN_INPUT 2
 #define PML_FLAG_PREPARE 4
+#define PML_FLAG_AUTO 8
 
 int pml_fdm_solve(int eq_id, const double *eq_params, int n_params,
                   int integrator_id, int precision, int ndim,

@@ -390,6 +390,7 @@ class FDMBatch:
         first_grid: int = 0,
         n_grids: Optional[int] = None,
         prepare: bool = False,
+        auto: bool = False,
     ) -> None:
         """Advances grids ``[first_grid, first_grid + n_grids)`` (default: all)
         by ``n_steps`` steps in place.  ``snapshots`` is an optional
@@ -397,7 +398,9 @@ class FDMBatch:
         every ``snapshot_every``-th step; ``constrain_input`` imposes the
         Dirichlet values on the state before the first step.  ``prepare``
         builds (and caches) the work-unit tables and the step-loop graph of
-        this call without launching anything."""
+        this call without launching anything.  ``auto`` lets the library take
+        the many-step kernel instead of ``tile_config`` where the batch is
+        small enough for it (same results)."""
         snap_hi = snap_lo = None
         if snapshots is not None:
             snap_hi, snap_lo = snapshots
@@ -426,7 +429,8 @@ class FDMBatch:
                 int(tile_config),
                 (nat.PML_FLAG_GRAPH if use_graph else 0)
                 | (nat.PML_FLAG_CONSTRAIN_INPUT if constrain_input else 0)
-                | (nat.PML_FLAG_PREPARE if prepare else 0),
+                | (nat.PML_FLAG_PREPARE if prepare else 0)
+                | (nat.PML_FLAG_AUTO if auto else 0),
                 self._sptr(),
             )
         )

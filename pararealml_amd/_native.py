@@ -37,6 +37,7 @@ PML_JACOBI_STATE_BYTES = 32 + 8 * PML_REDUCE_SLOTS
 PML_FLAG_GRAPH = 1
 PML_FLAG_CONSTRAIN_INPUT = 2
 PML_FLAG_PREPARE = 4
+PML_FLAG_AUTO = 8
 
 PML_INT_FE = 0
 PML_INT_MIDPOINT = 1

@@ -87,6 +87,12 @@ def lookup(problem, integrator: int, precision: str, cells: Optional[int] = None
         return 0
 
 
+def recorded(problem, integrator: int, precision: str, cells: Optional[int] = None) -> bool:
+    """Whether a tuning run recorded a variant for this key."""
+    with _lock:
+        return key_for(problem, integrator, precision, cells) in _load()
+
+
 def tune(batch, d_t: float, n_steps: int = 64, repeats: int = 3, store: bool = True):
     """Times every variant on ``batch`` (an ``FDMBatch``; its state is
     advanced and therefore clobbered) and records the fastest.  Returns

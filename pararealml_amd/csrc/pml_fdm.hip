@@ -9,7 +9,7 @@
 #include <string>
 #include <vector>
 
-#include "pml_fdm_kernels.h"
+#include "pml_fdm_deep.h"
 
 namespace pml {
 
@@ -34,6 +34,83 @@ static const std::vector<Variant> *find_variants(int eq, int integ, int prec, in
     if (v) return v;
   }
   return nullptr;
+}
+
+static Deep find_deep(int eq, int integ, int prec, int ndim) {
+  if (prec == PML_F64) return fdm_deep_f64(eq, integ, ndim);
+  if (prec == PML_F32) return fdm_deep_f32(eq, integ, ndim);
+  return fdm_deep_f32c(eq, integ, ndim);
+}
+
+// How the many-step kernel would run a batch: output tiles of oy x ox with a
+// halo of `halo`, `steps` steps a launch (0: the streaming kernels run it).
+struct DeepPlan {
+  int oy = 0, ox = 0, halo = 0, steps = 0;
+};
+
+// One launch's steps at most (some 10 ms of a grid that fits one region) and
+// the tiles up to which the many-step kernel runs a batch: two and a half
+// rounds of one workgroup per CU, the most measured.
+constexpr int kDeepSteps = 2048;
+constexpr int64_t kDeepTiles = 640;
+
+// The plan with the least time a step by a model of the launches: 4.5 us a
+// launch, one workgroup a CU, and per stage 0.25 us (barrier, LDS round trip)
+// plus 0.17 us (FP64; 0.12 in FP32) per 1024 vertices and unit of arithmetic,
+// a unit being the diffusion equation's.  Measured against the default and
+// the best of the streaming variants, us a step (RK4 unless stated):
+//   FP64 diffusion FE 101 x 101   4.9 / 1.7 -> 1.0   600 x 600 5.0 / 2.1 -> 2.5
+//   FP64 diffusion 33 x 33       11.9 / 7.1 -> 1.9   600 x 600 11.0 / 8.4 -> 9.1
+//   FP64 Burgers, 500 on a line   6.6 / 5.7 -> 1.3   300 x 300 29.8 / 15.0 -> 8.2
+//   FP32 shallow water 513 x 385 29.8 / 16.6 -> 13.7 600 x 600 30.3 / 20.8 -> 18.8
+//   FP32 Cahn-Hilliard 300 x 300  6.5 / 2.2 -> 1.5   600 x 600 6.5 / 2.7 -> 2.8
+// Regions above 1024 vertices hold two a thread, which three fields (and two
+// with first derivatives in FP64) have no registers for.
+static DeepPlan deep_plan(const Deep &d, const pml_grid *grids, int n_grids, int ndim,
+                          int64_t n_steps) {
+  DeepPlan best;
+  double best_us = 0.0;
+  if (!d.fn[0] || n_steps < 2) return best;
+  int64_t whole = 0;  // the largest grid's vertices
+  int max0 = 1, max1 = 1;
+  for (int g = 0; g < n_grids; ++g) {
+    whole = std::max(whole, static_cast<int64_t>(grids[g].n0) * grids[g].n1);
+    max0 = std::max(max0, grids[g].n0);
+    max1 = std::max(max1, grids[g].n1);
+  }
+  auto consider = [&](int oy, int ox, int halo, int steps, int64_t region) {
+    if (region > d.most || 2 * static_cast<int64_t>(d.fields) * region * d.value_bytes > kDeepLds)
+      return;
+    int64_t tiles = 0;
+    for (int g = 0; g < n_grids; ++g)
+      tiles += static_cast<int64_t>((grids[g].n0 + oy - 1) / oy) * ((grids[g].n1 + ox - 1) / ox);
+    if (tiles > kDeepTiles) return;
+    const double stage_us =
+        0.25 + (d.value_bytes == 8 ? 0.17 : 0.12) * d.units * static_cast<double>(region) / 1024.0;
+    const double launch_us = 4.5 + (tiles + 255) / 256 * (steps * d.stages * stage_us);
+    if (!best.steps || launch_us / steps < best_us) {
+      best.oy = oy;
+      best.ox = ox;
+      best.halo = halo;
+      best.steps = steps;
+      best_us = launch_us / steps;
+    }
+  };
+  const int most_steps = static_cast<int>(std::min<int64_t>(n_steps, kDeepSteps));
+  consider(max0, max1, 0, most_steps, whole);
+  // halos of whole steps: 8 and 4 vertices in 2-D, 96 on a line
+  for (int halo : {8, 4, 96}) {
+    if ((halo == 96) != (ndim == 1)) continue;
+    const int steps = std::min(halo / d.stages, most_steps), need = steps * d.stages;
+    if (ndim == 1) {
+      consider(1, 256, need, steps, std::min<int64_t>(max1, 256 + 2 * need));
+      continue;
+    }
+    for (int o : {16, 24, 32})
+      consider(o, o, need, steps,
+               std::min<int64_t>(max0, o + 2 * need) * std::min<int64_t>(max1, o + 2 * need));
+  }
+  return best;
 }
 
 // Device copies of work-unit and grid tables.  They are derived from the
@@ -331,6 +408,86 @@ static int fdm_solve_impl(int eq_id, const double *eq_params, int n_params,
       return fail(PML_E_INVALID, "a single grid must hold fewer than 2^31 values");
   }
   hipStream_t st = as_stream(stream);
+  // Dirichlet values imposed on the input state in place (it is overwritten
+  // by the result anyway).
+  auto constrain_input = [&](const void *grid_table) -> int {
+    const dim3 cgrid(n_grids, n_fields);
+    const auto *gd = static_cast<const GridDev *>(grid_table);
+    if (precision == PML_F64)
+      hipLaunchKernelGGL(fdm_constrain<PrecF64>, cgrid, dim3(256), 0, st, gd, bc_values, state_hi,
+                         state_lo, ndim);
+    else if (precision == PML_F32C)
+      hipLaunchKernelGGL(fdm_constrain<PrecF32C>, cgrid, dim3(256), 0, st, gd, bc_values,
+                         state_hi, state_lo, ndim);
+    else
+      hipLaunchKernelGGL(fdm_constrain<PrecF32>, cgrid, dim3(256), 0, st, gd, bc_values, state_hi,
+                         state_lo, ndim);
+    PML_LAUNCH_CHECK();
+    return PML_OK;
+  };
+  if ((flags & PML_FLAG_AUTO) && !no_alloc && !leave) {
+    const Deep deep = find_deep(eq_id, integrator_id, precision, ndim);
+    const DeepPlan plan = deep_plan(deep, grids, n_grids, ndim, n_steps);
+    if (plan.steps) {
+      Variant shape{};
+      shape.ox = plan.ox;
+      shape.oy = plan.oy;
+      TableSet tab;
+      if (int rc = device_tables(grids, n_grids, shape, ndim, &tab); rc != PML_OK) return rc;
+      if (prepare) return PML_OK;
+      if (constrain)
+        if (int rc = constrain_input(tab.grids); rc != PML_OK) return rc;
+      int64_t cells = 0;  // of the largest region
+      for (int g = 0; g < n_grids; ++g) {
+        const int64_t h = std::min(grids[g].n0, plan.oy + 2 * plan.halo);
+        const int64_t w = std::min(grids[g].n1, plan.ox + 2 * plan.halo);
+        cells = std::max(cells, h * w);
+      }
+      const DeepFn fn = deep.fn[cells > kDeepThreads];
+      const int threads =
+          static_cast<int>(std::min<int64_t>(kDeepThreads, (cells + 63) / 64 * 64));
+      const size_t lds = deep.lds(cells);
+      PML_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, kDeepLds));
+      DeepArgs a{};
+      a.tiles = static_cast<const TileDev *>(tab.units);
+      a.grids = static_cast<const GridDev *>(tab.grids);
+      a.bc = bc_values;
+      void *cur_hi = state_hi, *cur_lo = state_lo, *nxt_hi = work_hi, *nxt_lo = work_lo;
+      a.snap_hi = snapshots_hi;
+      a.snap_lo = snapshots_lo;
+      a.dt = dt;
+      for (int i = 0; i < 6; ++i) a.p[i] = i < n_params ? eq_params[i] : 0.0;
+      a.total = total_elems;
+      a.snap_every = static_cast<int>(
+          std::min<int64_t>(snapshots_hi ? snapshot_every : n_steps + 1, 1 << 30));
+      a.n_tiles = tab.n_units;
+      a.ndim = ndim;
+      a.oy = plan.oy;
+      a.ox = plan.ox;
+      a.halo = plan.halo;
+      for (int64_t done = 0; done < n_steps; done += a.steps) {
+        a.steps = static_cast<int>(std::min<int64_t>(plan.steps, n_steps - done));
+        a.in_hi = cur_hi;
+        a.in_lo = cur_lo;
+        a.out_hi = nxt_hi;
+        a.out_lo = nxt_lo;
+        a.snap_idx = done / a.snap_every;
+        a.until = static_cast<int>(a.snap_every - done % a.snap_every);
+        hipLaunchKernelGGL(fn, dim3(tab.n_units), dim3(threads), lds, st, a);
+        PML_LAUNCH_CHECK();
+        std::swap(cur_hi, nxt_hi);
+        std::swap(cur_lo, nxt_lo);
+      }
+      if (cur_hi != state_hi) {
+        const size_t bytes = total_elems * (precision == PML_F64 ? 8 : 4);
+        PML_HIP_CHECK(hipMemcpyAsync(state_hi, cur_hi, bytes, hipMemcpyDeviceToDevice, st));
+        if (precision == PML_F32C)
+          PML_HIP_CHECK(hipMemcpyAsync(state_lo, cur_lo, bytes, hipMemcpyDeviceToDevice, st));
+      }
+      return PML_OK;
+    }
+  }
   TableSet tab;
   if (no_alloc && (flags & PML_FLAG_PREPARE))
     return fail(PML_E_INVALID, "the allocation-free entry point has nothing to prepare");
@@ -382,21 +539,8 @@ static int fdm_solve_impl(int eq_id, const double *eq_params, int n_params,
   const int64_t fused_launches = n_steps / steps_per_launch;
   if (prepare && !(graphed && fused_launches >= 2)) return PML_OK;  // tables only
 
-  // Dirichlet values imposed on the input state in place (it is overwritten
-  // by the result anyway).
-  if (constrain && n_steps > 0 && !prepare) {
-    const dim3 cgrid(n_grids, n_fields);
-    if (precision == PML_F64)
-      hipLaunchKernelGGL(fdm_constrain<PrecF64>, cgrid, dim3(256), 0, st, a.grids, bc_values,
-                         state_hi, state_lo, ndim);
-    else if (precision == PML_F32C)
-      hipLaunchKernelGGL(fdm_constrain<PrecF32C>, cgrid, dim3(256), 0, st, a.grids, bc_values,
-                         state_hi, state_lo, ndim);
-    else
-      hipLaunchKernelGGL(fdm_constrain<PrecF32>, cgrid, dim3(256), 0, st, a.grids, bc_values,
-                         state_hi, state_lo, ndim);
-    PML_LAUNCH_CHECK();
-  }
+  if (constrain && n_steps > 0 && !prepare)
+    if (rc = constrain_input(a.grids); rc != PML_OK) return rc;
 
   int64_t li = 0;
 

@@ -1674,6 +1674,58 @@ __global__ __launch_bounds__(256) void fdm_constrain(const GridDev *grids, const
   }
 }
 
+// What field f of a cell becomes in stage `stage` (0-based), where k is the
+// stage's time step (half of it in the midpoint method's first stage) times
+// the right-hand side, alg the algebraic value from the pre-step state and
+// (yh, yl) the step's start, which the last stage turns into its result; acc
+// is the Runge-Kutta sum.  Returns the next stage's input or the result.
+template <class Eq, class Integ, class P>
+__device__ __forceinline__ typename P::C stage_update(int f, int stage, typename P::C k,
+                                                      typename P::C alg, typename P::C &yh,
+                                                      typename P::C &yl, typename P::C &acc) {
+  using C = typename P::C;
+  constexpr int S = Eq::kInvariant ? 1 : Integ::kStages;
+  const bool last = stage == S - 1;
+  if ((Eq::kAlg >> f) & 1u) {
+    if (last) {
+      yh = alg;
+      yl = 0;
+    }
+    return yh;
+  }
+  if (Eq::kInvariant) {
+    C d = k;
+    if (Integ::kStages == 4) d = (fma_pow2(C(2), k, fma_pow2(C(2), k, k)) + k) * C(1.0 / 6.0);
+    state_add<P>(yh, yl, d);
+    return yh;
+  }
+  if (Integ::kStages == 1) {
+    state_add<P>(yh, yl, k);
+    return yh;
+  }
+  if (Integ::kStages == 2) {
+    if (stage == 0) return state_plus<P>(yh, yl, k);
+    state_add<P>(yh, yl, k);
+    return yh;
+  }
+  // RK4
+  if (stage == 0) {
+    acc = k;
+    return state_plus_half<P>(yh, yl, k);
+  }
+  if (stage == 1) {
+    acc = fma_pow2(C(2), k, acc);
+    return state_plus_half<P>(yh, yl, k);
+  }
+  if (stage == 2) {
+    acc = fma_pow2(C(2), k, acc);
+    return state_plus<P>(yh, yl, k);
+  }
+  acc = acc + k;
+  state_add<P>(yh, yl, acc * C(1.0 / 6.0));
+  return yh;
+}
+
 // ---------------------------------------------------------------------------
 // fdm_fused: LDS tiles with shrinking stage regions, STEPS steps per launch.
 template <class Eq, class Integ, class P, int OX, int OY, int STEPS, int NT>
@@ -1791,46 +1843,9 @@ __global__ __launch_bounds__(NT) void fdm_fused(FdmArgs a) {
 #pragma unroll
           for (int f = 0; f < F; ++f) {
             const bool alg = (Eq::kAlg >> f) & 1u;
-            C nv;  // new LDS value (stage input, or the step result)
-            if (alg) {
-              if (last) {
-                yh[k][f] = an[k][f];
-                yl[k][f] = 0;
-              }
-              nv = yh[k][f];
-            } else if (Eq::kInvariant) {
-              const C kk = kn[k][f];
-              C d = kk;
-              if (Integ::kStages == 4) d = (fma_pow2(C(2), kk, fma_pow2(C(2), kk, kk)) + kk) * C(1.0 / 6.0);
-              state_add<P>(yh[k][f], yl[k][f], d);
-              nv = yh[k][f];
-            } else if (Integ::kStages == 1) {
-              state_add<P>(yh[k][f], yl[k][f], kn[k][f]);
-              nv = yh[k][f];
-            } else if (Integ::kStages == 2) {
-              if (stage == 0) {
-                nv = state_plus<P>(yh[k][f], yl[k][f], kn[k][f]);
-              } else {
-                state_add<P>(yh[k][f], yl[k][f], kn[k][f]);
-                nv = yh[k][f];
-              }
-            } else {  // RK4
-              const C kk = kn[k][f];
-              if (stage == 0) {
-                kacc[k][f] = kk;
-                nv = state_plus_half<P>(yh[k][f], yl[k][f], kk);
-              } else if (stage == 1) {
-                kacc[k][f] = fma_pow2(C(2), kk, kacc[k][f]);
-                nv = state_plus_half<P>(yh[k][f], yl[k][f], kk);
-              } else if (stage == 2) {
-                kacc[k][f] = fma_pow2(C(2), kk, kacc[k][f]);
-                nv = state_plus<P>(yh[k][f], yl[k][f], kk);
-              } else {
-                kacc[k][f] = kacc[k][f] + kk;
-                state_add<P>(yh[k][f], yl[k][f], kacc[k][f] * C(1.0 / 6.0));
-                nv = yh[k][f];
-              }
-            }
+            // new LDS value (stage input, or the step result)
+            C nv = stage_update<Eq, Integ, P>(f, stage, kn[k][f], an[k][f], yh[k][f], yl[k][f],
+                                              kacc[k][f]);
             if (edge) {
               const double dv = dirichlet_at(bcg + f * fstride, n0, n1, gi, gj, ax0);
               if (dv == dv) {

@@ -213,6 +213,17 @@ class FDMOperator(Operator):
         return lookup(problem, dev.integrator_id(self._integrator), self._precision,
                       cells=problem.plane * int(n_grids))
 
+    def kernel_choice(self, problem, n_grids: int = 1) -> dict:
+        """``FDMBatch.advance`` arguments for a batch of ``n_grids`` grids of
+        ``problem``: ``tile_config_for``, and ``auto`` where neither the
+        constructor nor a tuning run chose that variant."""
+        from pararealml_amd.autotune import recorded
+
+        chosen = self._tile_config is not None or recorded(
+            problem, dev.integrator_id(self._integrator), self._precision,
+            cells=problem.plane * int(n_grids))
+        return dict(tile_config=self.tile_config_for(problem, n_grids), auto=not chosen)
+
     def tune(self, cp, n_grids: int = 1, n_steps: int = 64, seed: int = 0) -> int:
         """Times every kernel variant on a scratch batch of ``n_grids``
         copies of ``cp``'s grid (random state, this operator's time step)
@@ -295,8 +306,8 @@ class FDMOperator(Operator):
                 n_steps,
                 snaps,
                 every,
-                tile_config=self.tile_config_for(problem),
                 use_graph=self._use_graph,
+                **self.kernel_choice(problem),
             )
             dev_y = batch.snapshots_f64(snaps, n_snap)
             y = dev.states_to_host(dev_y, problem, cp.mesh.vertices_shape)

@@ -372,7 +372,7 @@ def corrected_pairs(base_op, cp, snaps, slice_dt: float, stream=None, base_level
                 batch.load_f64(xb)
             else:
                 batch.load_f64(x.view(-1))
-            batch.advance(base_op.d_t, steps, tile_config=base_op.tile_config_for(bp, n),
+            batch.advance(base_op.d_t, steps, **base_op.kernel_choice(bp, n),
                           use_graph=True, constrain_input=True)
             yb = batch.state_f64()
             grids._dirichlet(yb.data_ptr(), base_levels, n, sp)
@@ -444,7 +444,7 @@ def generate_pairs(fdm_op, cp, y0s: np.ndarray, t_span: float, pair_dt: float,
         tmp = torch.empty((n * wp.n_fields, wp.n0, wp.n1), dtype=torch.float64, device="cuda")
         for k in range(n_pairs + 1):
             if k:
-                batch.advance(fdm_op.d_t, steps, tile_config=fdm_op.tile_config_for(problem, n),
+                batch.advance(fdm_op.d_t, steps, **fdm_op.kernel_choice(problem, n),
                               use_graph=True)
             batch.state_f64(f64)
             if lv:

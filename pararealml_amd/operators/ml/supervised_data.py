@@ -216,8 +216,7 @@ class SupervisedDataProtocol:
                 loaded = batch.state_f64()
                 snaps = batch.new_snapshots(n_snap) if n_snap else None
                 batch.advance(oracle.d_t, n_steps, snaps, every,
-                              tile_config=oracle.tile_config_for(problem, len(ys)),
-                              use_graph=True)
+                              use_graph=True, **oracle.kernel_choice(problem, len(ys)))
                 final = batch.state_f64()
                 out = (loaded.view(len(ys), -1), final.view(len(ys), -1))
                 if n_snap:

@@ -83,11 +83,11 @@ class FDMSlicePropagator:
             self.steps,
             snapshots=self.snaps,
             snapshot_every=1 if self.snaps is not None else 0,
-            tile_config=self.op.tile_config_for(self.problem, count),
             use_graph=True,
             constrain_input=True,
             first_grid=first,
             n_grids=count,
+            **self.op.kernel_choice(self.problem, count),
         )
         nat.check(lib.pml_to_f64(b.prec, hi, lo, out_f64.data_ptr(), count * self.elems,
                                  self._sptr()))
