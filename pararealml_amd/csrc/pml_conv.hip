@@ -5,9 +5,8 @@
 //    (v_mfma_f32_32x32x16_bf16).  Implicit GEMM: M = pixels, N = 64 output
 //    channels, K = 9 taps x 64 input channels.  A persistent workgroup of
 //    8 wavefronts keeps all 9 taps of the weights in LDS and loops over
-//    8 x 32-pixel output tiles; each wavefront computes one 32-pixel row
-//    of the tile against all 64 output channels (two 32x32 accumulator
-//    blocks).  The same main loop serves the forward pass (epilogue: bias,
+//    output tiles of 4 or 8 rows of 32 pixels; a pair of wavefronts computes
+//    one or two rows, 32 output channels each.  The same main loop serves the forward pass (epilogue: bias,
 //    GELU, BF16 pre-activation and activation) and the input gradient
 //    (weights pre-arranged flipped and transposed; epilogue: times GELU'
 //    of the previous layer's pre-activation).
@@ -54,8 +53,8 @@ __device__ __forceinline__ float gelu_grad_f(float z) {
 }
 
 // ---------------------------------------------------------------------------
-// conv64 (MFMA).  Output tile: kTR = 16 rows x kTC = 32 columns x 64
-// channels.  The input patch (18 x 34 pixels) sits in LDS as 144-byte rows
+// conv64 (MFMA).  Output tile: 4 R = 4 or 8 rows x kTC = 32 columns x 64
+// channels (the figures below for R = 2).  The input patch (10 x 34 pixels) sits in LDS as 144-byte rows
 // (64 BF16 channels + 16 bytes of padding: 16 lanes reading consecutive
 // rows hit all 64 banks once, and every patch address is a per-lane base
 // plus an immediate).  All nine taps of the weights sit beside it as
@@ -63,21 +62,22 @@ __device__ __forceinline__ float gelu_grad_f(float z) {
 // (row / 2) mod 8, which spreads any 16 consecutive rows over the 64 banks.
 // The MFMA's A operand is a weight block (32 output channels x 16 input
 // channels), B a pixel block (16 input channels x 32 pixels of one row).
-// Wavefront w owns output rows 4 (w / 2) .. + 3 and output channels
+// Wavefront w owns output rows 2 (w / 2) and the next and output channels
 // 32 (w % 2) .. + 31: for each tap column and 16-channel slice it reads the
-// six patch rows and the three kernel-row weight blocks those four rows need
-// once and issues 12 MFMAs.  The next tile's patch is loaded into registers
+// four patch rows and the three kernel-row weight blocks those rows need
+// once and issues 6 MFMAs.  The next tile's patch is loaded into registers
 // while the current one is computed.
-constexpr int kTR = 16, kTC = 32;
-constexpr int kPR = kTR + 2, kPC = kTC + 2;  // input patch incl. halo
-constexpr int kPatchPitch = 144;             // bytes per patch pixel
-constexpr int kPatchChunks = kPR * kPC * 8;  // 16-byte chunks
-constexpr int kPatchBytes = kPR * kPC * kPatchPitch;
+constexpr int kTC = 32;
+constexpr int kPC = kTC + 2;      // patch columns incl. halo
+constexpr int kPatchPitch = 144;  // bytes per patch pixel
 constexpr int kWBytes = 9 * 64 * 128;
-constexpr size_t kConvLds = kPatchBytes + kWBytes;
 constexpr int kConvThreads = 512;
-constexpr int kPrefetch = (kPatchChunks + kConvThreads - 1) / kConvThreads;
-static_assert(kConvLds <= 160 * 1024, "conv64 LDS budget");
+// Rows per wavefront R: the tile has 4 R rows, R = 2 or 1 (conv_rows()).
+constexpr int conv_patch_rows(int R) { return 4 * R + 2; }
+constexpr size_t conv_lds(int R) {
+  return static_cast<size_t>(conv_patch_rows(R)) * kPC * kPatchPitch + kWBytes;
+}
+static_assert(conv_lds(2) <= 160 * 1024, "conv64 LDS budget");
 
 // Byte offset of 16-byte chunk `chunk` (0..7) of weight row `row`.
 __device__ __forceinline__ int wswz(int row, int chunk) {
@@ -113,15 +113,18 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t conv_rsrc(const void *p, unsig
 struct TilePos {
   int b, h0, w0;
 };
+template <int R>
 __device__ __forceinline__ TilePos tile_pos(const ConvArgs &a, int tile) {
   const int per_img = a.tiles_h * a.tiles_w;
   const int b = tile / per_img;
   const int rem = tile - b * per_img;
-  return {b, (rem / a.tiles_w) * kTR, (rem % a.tiles_w) * kTC};
+  return {b, (rem / a.tiles_w) * 4 * R, (rem % a.tiles_w) * kTC};
 }
 
-template <int MODE>
+template <int MODE, int R>
 __global__ __launch_bounds__(kConvThreads) void k_conv64(ConvArgs a) {
+  constexpr int kPatchChunks = conv_patch_rows(R) * kPC * 8;  // 16-byte chunks
+  constexpr int kPrefetch = (kPatchChunks + kConvThreads - 1) / kConvThreads;
   extern __shared__ __align__(16) unsigned char smem[];
   unsigned char *wl = smem;
   unsigned char *patch = smem + kWBytes;
@@ -164,7 +167,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv64(ConvArgs a) {
   }
   u32x4 pre[kPrefetch];
   auto fetch = [&](int tile) {
-    const TilePos tp = tile_pos(a, tile);
+    const TilePos tp = tile_pos<R>(a, tile);
     const int origin = ((tp.b * a.H + tp.h0) * a.W + tp.w0) * 128;
 #pragma unroll
     for (int s = 0; s < kPrefetch; ++s) {
@@ -176,9 +179,9 @@ __global__ __launch_bounds__(kConvThreads) void k_conv64(ConvArgs a) {
     }
   };
 
-  // Per-lane LDS bases: patch pixel (4 rg, i) chunk kh, and weight row
+  // Per-lane LDS bases: patch pixel (R rg, i) chunk kh, and weight row
   // 32 nh + i of tap 0 for each 16-channel slice kc.
-  const int pbase = ((4 * rg) * kPC + i) * kPatchPitch + kh * 16;
+  const int pbase = ((R * rg) * kPC + i) * kPatchPitch + kh * 16;
   int wbase[4];
 #pragma unroll
   for (int kc = 0; kc < 4; ++kc) wbase[kc] = wswz(nh * 32 + i, 2 * kc + kh);
@@ -194,7 +197,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv64(ConvArgs a) {
         *reinterpret_cast<u32x4 *>(patch + (c >> 3) * kPatchPitch + (c & 7) * 16) = pre[s];
     }
     __syncthreads();
-    const TilePos tp = tile_pos(a, tile);
+    const TilePos tp = tile_pos<R>(a, tile);
     if (tile + static_cast<int>(gridDim.x) < a.n_tiles) fetch(tile + gridDim.x);
 
     // The two wavefronts sharing a SIMD (w and w + 4) run the MFMA phase
@@ -202,18 +205,18 @@ __global__ __launch_bounds__(kConvThreads) void k_conv64(ConvArgs a) {
     // runs its VALU epilogue while the second still issues MFMAs.
     if (wave < 4) __builtin_amdgcn_s_setprio(2);
     else __builtin_amdgcn_s_setprio(1);
-    f32x16 acc[4];
+    f32x16 acc[R];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < R; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[j][r] = bias[r];
     // 12 steps (tap column tw, 16-channel slice kc); the fragments of step
     // st + 1 are read while the MFMAs of step st run.
-    bf16x8 pv[2][6], wv[2][3];
-    auto load_step = [&](int st, bf16x8 (&p6)[6], bf16x8 (&w3)[3]) {
+    bf16x8 pv[2][R + 2], wv[2][3];
+    auto load_step = [&](int st, bf16x8 (&p6)[R + 2], bf16x8 (&w3)[3]) {
       const int tw = st >> 2, kc = st & 3;
 #pragma unroll
-      for (int r = 0; r < 6; ++r)
+      for (int r = 0; r < R + 2; ++r)
         p6[r] = *reinterpret_cast<const bf16x8 *>(patch + pbase + (r * kPC + tw) * kPatchPitch +
                                                   kc * 32);
 #pragma unroll
@@ -231,7 +234,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv64(ConvArgs a) {
 #pragma unroll
       for (int th = 0; th < 3; ++th)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < R; ++j)
           acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[cur][th], pv[cur][j + th], acc[j],
                                                            0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
@@ -242,24 +245,24 @@ __global__ __launch_bounds__(kConvThreads) void k_conv64(ConvArgs a) {
     // the image use the drop offset.  The backward pass issues all its
     // pre-activation loads before using any.
     const int w = tp.w0 + i;
-    unsigned base[4];
+    unsigned base[R];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int h = tp.h0 + 4 * rg + j;
+    for (int j = 0; j < R; ++j) {
+      const int h = tp.h0 + R * rg + j;
       base[j] = h < a.H && w < a.W
                     ? ((static_cast<unsigned>(tp.b * a.H + h) * a.W + w) * 64 + nh * 32 + 4 * kh) * 2
                     : kDrop;
     }
-    u32x2 zp[4][4];
+    u32x2 zp[R][4];
     if (MODE == kBwd) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < R; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           zp[j][q] = __builtin_amdgcn_raw_buffer_load_b64(r_z, base[j] + 16 * q, 0, 0);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < R; ++j) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         bf16x4 o4;
@@ -481,7 +484,16 @@ __global__ void k_sum_segments(const float *part, int n_blocks, int per_block, i
   if (i >= n) return;
   const int b0 = blockIdx.y * kSumSeg, b1 = min(b0 + kSumSeg, n_blocks);
   float s = 0.0f;
-  for (int b = b0; b < b1; ++b) s += part[static_cast<size_t>(b) * per_block + i];
+  // (the additions in block order, the loads of several rows at once: one
+  // after the other they cost a memory latency each)
+  for (int b = b0; b < b1; b += 8) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      v[k] = b + k < b1 ? part[static_cast<size_t>(b + k) * per_block + i] : 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += v[k];
+  }
   seg[static_cast<size_t>(blockIdx.y) * n + i] = s;
 }
 __global__ void k_sum_blocks(const float *seg, int n_segs, int n, float *dw, int n_dw,
@@ -489,7 +501,14 @@ __global__ void k_sum_blocks(const float *seg, int n_segs, int n, float *dw, int
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   float s = 0.0f;
-  for (int y = 0; y < n_segs; ++y) s += seg[static_cast<size_t>(y) * n + i];
+  for (int y = 0; y < n_segs; y += 8) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      v[k] = y + k < n_segs ? seg[static_cast<size_t>(y + k) * n + i] : 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += v[k];
+  }
   if (i < n_dw) dw[i] += s;
   else db[i - n_dw] += s;
 }
@@ -1058,6 +1077,31 @@ static int cu_count() {
 
 using namespace pml;
 
+template <int MODE, int R>
+static int launch_conv64(const ConvArgs &a, hipStream_t st) {
+  PML_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv64<MODE, R>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, conv_lds(R)));
+  hipLaunchKernelGGL((k_conv64<MODE, R>), dim3(std::min(a.n_tiles, cu_count())),
+                     dim3(kConvThreads), conv_lds(R), st, a);
+  PML_LAUNCH_CHECK();
+  return PML_OK;
+}
+
+// Rows per wavefront of a launch: the fewer rounds of one workgroup per CU,
+// a round taking 4.4 us with one row and 8 us with two (beside some 3 us for
+// the launch and the weights).  Measured forward, one row / two (with four
+// rows, as tiles of 16, before): 1 x 33 x 33 7.1 / 9.6 (14.5), 1 x 129 x 129
+// 7.9 / 10.4 (15.5), 1 x 257 x 129 11.8 / 11.1 (16.1), 4 x 129 x 129 16.9 /
+// 18.9 (18.5), 8 x 129 x 129 25.5 / 25.5 (30.8), 16 x 129 x 129 41.7 / 41.3
+// (41.5) us; the input gradient of the last 38.4 / 38.0 (39.9).
+static int conv_rows(int images, int H, int tiles_w) {
+  auto us = [&](int r) {
+    const int64_t tiles = static_cast<int64_t>(images) * ((H + 4 * r - 1) / (4 * r)) * tiles_w;
+    return static_cast<double>((tiles + cu_count() - 1) / cu_count()) * (0.8 + 3.6 * r);
+  };
+  return us(1) < us(2) ? 1 : 2;
+}
+
 extern "C" int pml_conv64(int mode, const void *in, const void *wk, const float *bias,
                           const void *zprev, void *z_out, void *a_out, int B, int H, int W,
                           void *stream) {
@@ -1073,9 +1117,6 @@ extern "C" int pml_conv64(int mode, const void *in, const void *wk, const float 
   const int64_t img_bytes = img_elems * 2;
   if (img_bytes >= (int64_t(1) << 31)) return fail(PML_E_INVALID, "image too large for conv64");
   const int per = static_cast<int>(std::max<int64_t>(1, ((int64_t(1) << 31) - 1) / img_bytes));
-  const void *kern = mode == kFwd ? reinterpret_cast<const void *>(&k_conv64<kFwd>)
-                                  : reinterpret_cast<const void *>(&k_conv64<kBwd>);
-  PML_HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, kConvLds));
   hipStream_t st = as_stream(stream);
   for (int b0 = 0; b0 < B; b0 += per) {
     const int nb = std::min(per, B - b0);
@@ -1090,16 +1131,15 @@ extern "C" int pml_conv64(int mode, const void *in, const void *wk, const float 
     a.B = nb;
     a.H = H;
     a.W = W;
-    a.tiles_h = (H + kTR - 1) / kTR;
     a.tiles_w = (W + kTC - 1) / kTC;
-    a.n_tiles = nb * a.tiles_h * a.tiles_w;
     a.bytes = static_cast<unsigned>(nb * img_bytes);
-    const int grid = std::min(a.n_tiles, cu_count());
-    if (mode == kFwd)
-      hipLaunchKernelGGL(k_conv64<kFwd>, dim3(grid), dim3(kConvThreads), kConvLds, st, a);
-    else
-      hipLaunchKernelGGL(k_conv64<kBwd>, dim3(grid), dim3(kConvThreads), kConvLds, st, a);
-    PML_LAUNCH_CHECK();
+    const int rows = conv_rows(nb, H, a.tiles_w);
+    a.tiles_h = (H + 4 * rows - 1) / (4 * rows);
+    a.n_tiles = nb * a.tiles_h * a.tiles_w;
+    const int rc = mode == kFwd
+                       ? (rows == 2 ? launch_conv64<kFwd, 2>(a, st) : launch_conv64<kFwd, 1>(a, st))
+                       : (rows == 2 ? launch_conv64<kBwd, 2>(a, st) : launch_conv64<kBwd, 1>(a, st));
+    if (rc) return rc;
   }
   return PML_OK;
 }
