@@ -54,8 +54,10 @@ struct DeepPlan {
 constexpr int kDeepSteps = 2048;
 constexpr int64_t kDeepTiles = 640;
 
-// The plan with the least time a step by a model of the launches: 4.5 us a
-// launch, one workgroup a CU, and per stage 0.25 us (barrier, LDS round trip)
+// The plan with the least time by a model of the launches: 4.5 us a launch,
+// one workgroup a CU, the copy back that an odd number of launches ends with
+// (4 us and its bytes at 4 TB/s; 20 steps on 257 x 257 are two launches of
+// ten for it, 26 us instead of 34), and per stage 0.25 us (barrier, LDS round trip)
 // plus 0.17 us (FP64; 0.12 in FP32) per 1024 vertices and unit of arithmetic,
 // a unit being the diffusion equation's.  Measured against the default and
 // the best of the streaming variants, us a step (RK4 unless stated):
@@ -65,16 +67,20 @@ constexpr int64_t kDeepTiles = 640;
 //   FP32 shallow water 513 x 385 29.8 / 16.6 -> 13.7 600 x 600 30.3 / 20.8 -> 18.8
 //   FP32 Cahn-Hilliard 300 x 300  6.5 / 2.2 -> 1.5   600 x 600 6.5 / 2.7 -> 2.8
 // Regions above 1024 vertices hold two a thread, which three fields (and two
-// with first derivatives in FP64) have no registers for.
+// with first derivatives in FP64) have no registers for; one such workgroup
+// fills a CU's registers, so they run one round only (FP64 wave 600 x 500 in
+// two-step regions of 1600: 13.0 us, in one-step ones of 1024: 11.0).
 static DeepPlan deep_plan(const Deep &d, const pml_grid *grids, int n_grids, int ndim,
                           int64_t n_steps) {
   DeepPlan best;
   double best_us = 0.0;
+  int64_t values = 0;  // of one state
   if (!d.fn[0] || n_steps < 2) return best;
   int64_t whole = 0;  // the largest grid's vertices
   int max0 = 1, max1 = 1;
   for (int g = 0; g < n_grids; ++g) {
     whole = std::max(whole, static_cast<int64_t>(grids[g].n0) * grids[g].n1);
+    values += static_cast<int64_t>(d.fields) * grids[g].n0 * grids[g].n1;
     max0 = std::max(max0, grids[g].n0);
     max1 = std::max(max1, grids[g].n1);
   }
@@ -84,24 +90,29 @@ static DeepPlan deep_plan(const Deep &d, const pml_grid *grids, int n_grids, int
     int64_t tiles = 0;
     for (int g = 0; g < n_grids; ++g)
       tiles += static_cast<int64_t>((grids[g].n0 + oy - 1) / oy) * ((grids[g].n1 + ox - 1) / ox);
-    if (tiles > kDeepTiles) return;
+    if (tiles > (region > kDeepThreads ? 256 : kDeepTiles)) return;
     const double stage_us =
         0.25 + (d.value_bytes == 8 ? 0.17 : 0.12) * d.units * static_cast<double>(region) / 1024.0;
-    const double launch_us = 4.5 + (tiles + 255) / 256 * (steps * d.stages * stage_us);
-    if (!best.steps || launch_us / steps < best_us) {
+    const int64_t launches = (n_steps + steps - 1) / steps;
+    double us = launches * 4.5 + (tiles + 255) / 256 * (n_steps * d.stages * stage_us);
+    if (launches & 1) us += 4.0 + 2.0 * values * d.value_bytes / 4e6;
+    if (!best.steps || us < best_us) {
       best.oy = oy;
       best.ox = ox;
       best.halo = halo;
       best.steps = steps;
-      best_us = launch_us / steps;
+      best_us = us;
     }
   };
   const int most_steps = static_cast<int>(std::min<int64_t>(n_steps, kDeepSteps));
   consider(max0, max1, 0, most_steps, whole);
-  // halos of whole steps: 8 and 4 vertices in 2-D, 96 on a line
-  for (int halo : {8, 4, 96}) {
+  // halos of whole steps, up to 4, 8 and 12 vertices in 2-D and 96 on a line,
+  // the steps shared out evenly over the launches
+  for (int halo : {4, 8, 12, 96}) {
     if ((halo == 96) != (ndim == 1)) continue;
-    const int steps = std::min(halo / d.stages, most_steps), need = steps * d.stages;
+    const int64_t launches = (n_steps + halo / d.stages - 1) / (halo / d.stages);
+    const int steps = static_cast<int>((n_steps + launches - 1) / launches);
+    const int need = steps * d.stages;
     if (ndim == 1) {
       consider(1, 256, need, steps, std::min<int64_t>(max1, 256 + 2 * need));
       continue;
