@@ -148,6 +148,9 @@ __global__ __launch_bounds__(kInterpBlock) void k_interp(
 // of up to 128).  Lanes run along t, so every corner read is one contiguous
 // run of the point's snapshots; the results pass through LDS (dynamic,
 // ts x 33 values) and leave as rows of 32 consecutive points per snapshot.
+// The rows are written past the caches, which keep the stack for the corner
+// reads of scattered points: 65 snapshots of 257 x 257 at 400000 points
+// 151.0 -> 143.3 us (the reads, 832 MB, come at 6 TB/s).
 constexpr int kTiPoints = 32;
 constexpr int kTiMaxSnaps = 128;
 
@@ -209,7 +212,9 @@ __global__ __launch_bounds__(kInterpBlock) void k_interp_ti(
     __syncthreads();
     for (int e = tid; e < t_loc * kTiPoints; e += kInterpBlock) {
       const int r = e / kTiPoints, q = e % kTiPoints;
-      if (q < n_loc) out[((t0 + r) * n_points + p0 + q) * C + c] = s_val[r * kRow + q];
+      if (q < n_loc)
+        __builtin_nontemporal_store(s_val[r * kRow + q],
+                                    &out[((t0 + r) * n_points + p0 + q) * C + c]);
     }
     __syncthreads();
   }
