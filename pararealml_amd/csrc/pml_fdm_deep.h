@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(kDeepThreads) fdm_deep(DeepArgs a) {
       from = to;
       to = t;
     }
-    if (--until == 0) {
+    if (--until == 0 && a.snap_hi) {
       write(a.snap_hi, a.snap_lo, snap * a.total);
       ++snap;
       until = a.snap_every;
