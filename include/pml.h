@@ -381,6 +381,25 @@ int pml_fdm_poisson_solve(int eq_id, const double *eq_params, int n_params,
                           void *jacobi_state, int64_t *sweeps_out, void *stream);
 
 /*
+ * One Parareal coarse solve on the 2x coarsened grid of a 2-D problem:
+ * fine_in (FP64, field-major, 2 m - 1 vertices an axis) injected into the
+ * coarse grid (*coarse, offsets 0, m >= 4; at most 32767 rows), n_steps steps
+ * there as by pml_fdm_solve (state, work: one coarse state each, in the given
+ * precision; flags: PML_FLAG_GRAPH, PML_FLAG_AUTO), and prolonged into
+ * fine_out as by pml_prolong2x_cubic; the Dirichlet values of coarse_bc and
+ * fine_bc (boundary blocks) are imposed on both grids.  Equals the calls
+ * pml_restrict2x, pml_apply_dirichlet, pml_from_f64, pml_fdm_solve,
+ * pml_to_f64, pml_prolong2x_cubic, pml_apply_dirichlet to the bit.
+ */
+int pml_fdm_coarse_step(int eq_id, const double *eq_params, int n_params,
+                        int integrator_id, int precision, const pml_grid *coarse,
+                        const double *coarse_bc, const double *fine_bc,
+                        const double *fine_in, double *fine_out, void *state_hi,
+                        void *state_lo, void *work_hi, void *work_lo,
+                        int64_t total_elems, double dt, int64_t n_steps,
+                        int tile_config, int flags, void *stream);
+
+/*
  * Results for the host.
  *   pml_channel_last: n_states field-major states (n_fields planes of `plane`
  *     FP64 values, 1 to 4 fields) -> channel-last copies.

@@ -38,6 +38,12 @@ int fail(int code, const std::string &msg);
 // Frees the pinned staging memory that pml_download keeps between calls.
 void release_staging();
 
+// The grid transfers of pml_fdm_coarse_step.
+int restrict_state(int precision, const double *fine, const double *bc, void *hi, void *lo,
+                   int n_fields, int m0, int m1, hipStream_t st);
+int prolong_state(int precision, const void *hi, const void *lo, const double *bc, double *fine,
+                  int n_fields, int m0, int m1, hipStream_t st);
+
 // One step of pml_fdm_solve from `in` into `out` (whole states, FP32 or FP64),
 // without the copy back that a call of an odd number of steps ends with.
 int fdm_step(int eq_id, const double *eq_params, int n_params, int integrator_id, int precision,

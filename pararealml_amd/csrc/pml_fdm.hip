@@ -716,3 +716,32 @@ extern "C" int pml_fdm_solve_noalloc(int eq_id, const double *eq_params, int n_p
                         dt, n_steps, snapshots_hi, snapshots_lo, snapshot_every, tile_config,
                         flags, stream, true);
 }
+
+extern "C" int pml_fdm_coarse_step(int eq_id, const double *eq_params, int n_params,
+                                   int integrator_id, int precision, const pml_grid *coarse,
+                                   const double *coarse_bc, const double *fine_bc,
+                                   const double *fine_in, double *fine_out, void *state_hi,
+                                   void *state_lo, void *work_hi, void *work_lo,
+                                   int64_t total_elems, double dt, int64_t n_steps,
+                                   int tile_config, int flags, void *stream) {
+  if (!coarse || !coarse_bc || !fine_bc || !fine_in || !fine_out || !state_hi || n_steps < 0 ||
+      (precision == PML_F32C && !state_lo))
+    return fail(PML_E_INVALID, "bad coarse step arguments");
+  int n_fields = 0;
+  if (!find_variants(eq_id, integrator_id, precision, 2, &n_fields))
+    return fail(PML_E_UNSUPPORTED, "no device kernel for this equation/integrator/precision");
+  const int m0 = coarse->n0, m1 = coarse->n1;
+  if (m0 < 4 || m1 < 4 || m0 > 32767 || m1 > (1 << 29) || coarse->state_offset != 0 ||
+      coarse->bc_offset != 0 ||
+      static_cast<int64_t>(n_fields) * m0 * m1 != total_elems)
+    return fail(PML_E_INVALID, "a coarse step takes one 2-D grid of at least 4 x 4 vertices");
+  hipStream_t st = as_stream(stream);
+  int rc = restrict_state(precision, fine_in, coarse_bc, state_hi, state_lo, n_fields, m0, m1, st);
+  if (rc) return rc;
+  rc = fdm_solve_impl(eq_id, eq_params, n_params, integrator_id, precision, 2, coarse, 1,
+                      coarse_bc, state_hi, state_lo, work_hi, work_lo, total_elems, dt, n_steps,
+                      nullptr, nullptr, 0, tile_config,
+                      flags & (PML_FLAG_GRAPH | PML_FLAG_AUTO), stream, false);
+  if (rc) return rc;
+  return prolong_state(precision, state_hi, state_lo, fine_bc, fine_out, n_fields, m0, m1, st);
+}

@@ -288,8 +288,35 @@ class CoarseGridPropagator:
         self.c_in = torch.empty(self.inner.elems, dtype=torch.float64, device="cuda")
         self.c_out = torch.empty(self.inner.elems, dtype=torch.float64, device="cuda")
         self.elems = self.grids.probs[0].elems
+        self._fused = self._fused_solve()
+
+    def _fused_solve(self):
+        """``(u, out) -> None``: one state's solve in one call
+        (``pml_fdm_coarse_step``), or None where it does not apply (several
+        levels, bilinear prolongation, fewer than 4 coarse vertices)."""
+        p, b = self.grids.probs[-1], self.inner.batch
+        if self.levels != 1 or self.grids.prolongation != "cubic" or p.ndim != 2 \
+                or min(p.n0, p.n1) < 4 or p.n0 > 32767:
+            return None
+        choice = self.inner.op.kernel_choice(p)
+        flags = nat.PML_FLAG_GRAPH | (nat.PML_FLAG_AUTO if choice["auto"] else 0)
+        ptr = b._ptr
+        head = (b.eq_id, b._params, len(b.params), b.integrator, b.prec, b.grids[0],
+                b.bc.data_ptr(), self.grids.bcs[0].data_ptr())
+        tail = (ptr(b.hi), ptr(b.lo), ptr(b.work_hi), ptr(b.work_lo), b.total,
+                float(self.inner.op.d_t), self.inner.steps, choice["tile_config"], flags,
+                self.stream.cuda_stream)
+
+        def solve(u, out):
+            nat.check(b.lib.pml_fdm_coarse_step(*head, u.data_ptr(), out.data_ptr(), *tail))
+
+        return solve
 
     def run(self, u_f64, first: int, last: int, out_f64):
+        if self._fused is not None:
+            for k in range(last - first):
+                self._fused(u_f64[k], out_f64[k])
+            return
         sp = ctypes.c_void_p(self.stream.cuda_stream)
         for k in range(last - first):
             self.grids.down(u_f64[k].data_ptr(), self.c_in.data_ptr(), 1, 0, self.levels, sp)
