@@ -365,15 +365,16 @@ int pml_laplacian_solve(int precision, int integrator_id, const int64_t *shape,
  * a device buffer of PML_JACOBI_STATE_BYTES.  *sweeps_out = the last solve's
  * sweeps, or 0 where the grid is too large for the device loop (nothing was
  * done) or a solve needs more than 16384 sweeps (state and snapshots are then
- * unspecified) or there was no step: step with
- * pml_fdm_solve and pml_jacobi_solve instead.  PML_F64 and PML_F32.
+ * unspecified) or there was no step: step with pml_fdm_solve and
+ * pml_jacobi_solve instead.  flags: PML_FLAG_AUTO.  PML_F64 and PML_F32.
  */
 int pml_fdm_poisson_solve(int eq_id, const double *eq_params, int n_params,
                           int integrator_id, int precision, const pml_grid *grid,
                           const double *bc_values, void *state, void *work,
                           int64_t total_elems, double dt, int64_t n_steps,
-                          int tile_config, int n_poisson, const int *field,
-                          const int *source, const double *scale,
+                          int tile_config, int flags, int n_poisson,
+                          const int *field, const int *source,
+                          const double *scale,
                           const double *const *ghost_lo,
                           const double *const *ghost_hi,
                           const double *const *ycons, double tol,

@@ -172,8 +172,8 @@ SIGNATURES = {
     "pml_fdm_poisson_solve": (
         c_int,
         [c_int, POINTER(c_double), c_int, c_int, c_int, POINTER(PmlGrid), c_void_p, c_void_p,
-         c_void_p, c_int64, c_double, c_int64, c_int, c_int, POINTER(c_int), POINTER(c_int),
-         POINTER(c_double), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), c_double,
+         c_void_p, c_int64, c_double, c_int64, c_int, c_int, c_int, POINTER(c_int),
+         POINTER(c_int), POINTER(c_double), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), c_double,
          c_void_p, c_int64, c_void_p, POINTER(c_int64), c_void_p],
     ),
     "pml_fdm_coarse_step": (

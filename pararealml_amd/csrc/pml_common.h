@@ -48,7 +48,7 @@ int prolong_state(int precision, const void *hi, const void *lo, const double *b
 // without the copy back that a call of an odd number of steps ends with.
 int fdm_step(int eq_id, const double *eq_params, int n_params, int integrator_id, int precision,
              int ndim, const pml_grid *grids, int n_grids, const double *bc_values, void *in,
-             void *out, int64_t total_elems, double dt, int tile_config, void *stream);
+             void *out, int64_t total_elems, double dt, int tile_config, int flags, void *stream);
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 

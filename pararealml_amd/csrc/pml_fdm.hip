@@ -66,6 +66,8 @@ constexpr int64_t kDeepTiles = 640;
 //   FP64 Burgers, 500 on a line   6.6 / 5.7 -> 1.3   300 x 300 29.8 / 15.0 -> 8.2
 //   FP32 shallow water 513 x 385 29.8 / 16.6 -> 13.7 600 x 600 30.3 / 20.8 -> 18.8
 //   FP32 Cahn-Hilliard 300 x 300  6.5 / 2.2 -> 1.5   600 x 600 6.5 / 2.7 -> 2.8
+// A single step gains the latency alone (the step of a lid-driven cavity's time
+// loop on 65 x 65: the 60-step run 1.80 -> 1.54 ms).
 // Regions above 1024 vertices hold two a thread, which three fields (and two
 // with first derivatives in FP64) have no registers for; one such workgroup
 // fills a CU's registers, so they run one round only (FP64 wave 600 x 500 in
@@ -75,7 +77,7 @@ static DeepPlan deep_plan(const Deep &d, const pml_grid *grids, int n_grids, int
   DeepPlan best;
   double best_us = 0.0;
   int64_t values = 0;  // of one state
-  if (!d.fn[0] || n_steps < 2) return best;
+  if (!d.fn[0] || n_steps < 1) return best;
   int64_t whole = 0;  // the largest grid's vertices
   int max0 = 1, max1 = 1;
   for (int g = 0; g < n_grids; ++g) {
@@ -436,7 +438,7 @@ static int fdm_solve_impl(int eq_id, const double *eq_params, int n_params,
     PML_LAUNCH_CHECK();
     return PML_OK;
   };
-  if ((flags & PML_FLAG_AUTO) && !no_alloc && !leave) {
+  if ((flags & PML_FLAG_AUTO) && !no_alloc) {
     const Deep deep = find_deep(eq_id, integrator_id, precision, ndim);
     const DeepPlan plan = deep_plan(deep, grids, n_grids, ndim, n_steps);
     if (plan.steps) {
@@ -490,7 +492,7 @@ static int fdm_solve_impl(int eq_id, const double *eq_params, int n_params,
         std::swap(cur_hi, nxt_hi);
         std::swap(cur_lo, nxt_lo);
       }
-      if (cur_hi != state_hi) {
+      if (cur_hi != state_hi && !leave) {
         const size_t bytes = total_elems * (precision == PML_F64 ? 8 : 4);
         PML_HIP_CHECK(hipMemcpyAsync(state_hi, cur_hi, bytes, hipMemcpyDeviceToDevice, st));
         if (precision == PML_F32C)
@@ -682,10 +684,11 @@ static int fdm_solve_impl(int eq_id, const double *eq_params, int n_params,
 
 int fdm_step(int eq_id, const double *eq_params, int n_params, int integrator_id, int precision,
              int ndim, const pml_grid *grids, int n_grids, const double *bc_values, void *in,
-             void *out, int64_t total_elems, double dt, int tile_config, void *stream) {
+             void *out, int64_t total_elems, double dt, int tile_config, int flags,
+             void *stream) {
   return fdm_solve_impl(eq_id, eq_params, n_params, integrator_id, precision, ndim, grids,
                         n_grids, bc_values, in, nullptr, out, nullptr, total_elems, dt, 1,
-                        nullptr, nullptr, 0, tile_config, 0, stream, false, true);
+                        nullptr, nullptr, 0, tile_config, flags, stream, false, true);
 }
 
 }  // namespace pml

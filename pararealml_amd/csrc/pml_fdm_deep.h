@@ -245,6 +245,7 @@ Deep deep_table(int eq, int integ, int ndim) {
     case PML_EQ_BURGERS:
       return ndim == 1 ? deep_by_int<EqBurgers1, PR>(integ) : deep_by_int<EqBurgers2, PR>(integ);
     case PML_EQ_SHALLOW_WATER: return deep_by_int<EqShallowWater, PR>(integ);
+    case PML_EQ_NAVIER_STOKES: return deep_by_int<EqNavierStokes, PR>(integ);
     default: return Deep{};
   }
 }

@@ -982,7 +982,8 @@ extern "C" int pml_fdm_poisson_solve(int eq_id, const double *eq_params, int n_p
                                      int integrator_id, int precision, const pml_grid *grid,
                                      const double *bc_values, void *state, void *work,
                                      int64_t total_elems, double dt, int64_t n_steps,
-                                     int tile_config, int n_poisson, const int *field,
+                                     int tile_config, int flags, int n_poisson,
+                                     const int *field,
                                      const int *source, const double *scale,
                                      const double *const *ghost_lo,
                                      const double *const *ghost_hi, const double *const *ycons,
@@ -1020,7 +1021,8 @@ extern "C" int pml_fdm_poisson_solve(int eq_id, const double *eq_params, int n_p
   char *cur = static_cast<char *>(state), *nxt = static_cast<char *>(work);
   for (int64_t s = 0; s < n_steps; ++s) {
     if (int rc = fdm_step(eq_id, eq_params, n_params, integrator_id, precision, 2, grid, 1,
-                          bc_values, cur, nxt, total_elems, dt, tile_config, stream);
+                          bc_values, cur, nxt, total_elems, dt, tile_config,
+                          flags & PML_FLAG_AUTO, stream);
         rc != PML_OK)
       return rc;
     for (int k = 0; k < n_poisson; ++k) {

@@ -860,7 +860,7 @@ class FDMOperator(Operator):
         return DeviceSolution(ivp, t[every::every], out, dev_y, vertex_oriented=True,
                               d_t=dt * every, copy=False)
 
-    def _poisson_loop(self, batch, problem, y_cons, d_cons, tile, n_steps, traj, every) -> bool:
+    def _poisson_loop(self, batch, problem, y_cons, d_cons, n_steps, traj, every) -> bool:
         """The whole time loop on the device (``pml_fdm_poisson_solve``);
         False where it does not cover the run, which then has to be stepped
         from its initial state."""
@@ -890,12 +890,14 @@ class FDMOperator(Operator):
             fixed.append(c)
         jacobi = torch.empty(nat.PML_JACOBI_STATE_BYTES // 8, dtype=torch.float64, device="cuda")
         sweeps = ctypes.c_int64(0)
+        choice = self.kernel_choice(problem)
         pointers = lambda ts: (ctypes.c_void_p * len(ts))(  # noqa: E731
             *[None if a is None else a.data_ptr() for a in ts])
         nat.check(batch.lib.pml_fdm_poisson_solve(
             batch.eq_id, batch._params, len(batch.params), batch.integrator, batch.prec,
             ctypes.byref(batch.grids[0]), batch.bc.data_ptr(), batch.hi.data_ptr(),
-            batch.work_hi.data_ptr(), batch.total, float(self._d_t), int(n_steps), int(tile), n,
+            batch.work_hi.data_ptr(), batch.total, float(self._d_t), int(n_steps),
+            choice["tile_config"], nat.PML_FLAG_AUTO if choice["auto"] else 0, n,
             (ctypes.c_int * n)(*[f for f, _, _ in problem.y_laplacian]),
             (ctypes.c_int * n)(*[src for _, src, _ in problem.y_laplacian]),
             (ctypes.c_double * n)(*[c for _, _, c in problem.y_laplacian]),
@@ -940,7 +942,7 @@ class FDMOperator(Operator):
             traj = torch.empty((n_snap, problem.elems), dtype=torch.float64, device="cuda")
             tile = self.tile_config_for(problem)
             state = batch.hi  # field-major, the batch precision
-            fused = self._poisson_loop(batch, problem, y_cons, d_cons, tile, n_steps, traj, every)
+            fused = self._poisson_loop(batch, problem, y_cons, d_cons, n_steps, traj, every)
             if not fused:  # a large grid, or a solve of many sweeps
                 batch.load_host([y0])
             for i in range(0 if fused else n_steps):

@@ -94,3 +94,30 @@ def test_many_step_kernel_on_ragged_batches():
 
 def test_large_batches_keep_their_variant():
     _compare("diffusion", [(700, 700)], 2, "float32", 3, 0)  # above 640 tiles
+
+
+@pytest.mark.parametrize("precision", ["float64", "float32"])
+@pytest.mark.parametrize("integ", [0, 1, 2])
+@pytest.mark.parametrize("n", [4, 31, 65, 129])
+def test_navier_stokes_single_steps(n, integ, precision):
+    """The step inside a Poisson time loop: algebraic fields, one step a
+    launch."""
+    import torch
+
+    from pararealml_amd import _device as dev
+    from tests.helpers import navier_stokes_cavity
+
+    print(f"case: deep navier-stokes {n} {integ} {precision}", flush=True)
+    cp, y0 = navier_stokes_cavity(n, re=100.0)
+    y0 = y0 + np.random.RandomState(n).uniform(-0.5, 0.5, y0.shape)
+    problem = dev.device_problem(cp)
+    stream = dev.solver_stream()
+    outs = []
+    with torch.cuda.stream(stream):
+        for auto in (False, True):
+            b = dev.FDMBatch([problem], [0], precision, integ, stream, poisson_phase=True)
+            b.load_host([y0])
+            for _ in range(3):
+                b.advance(D_T, 1, auto=auto)
+            outs.append(b.state_f64().cpu().numpy())
+    assert np.all(np.isfinite(outs[0])) and np.array_equal(*outs)
