@@ -5,7 +5,9 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstddef>
+#include <limits>
 #include <type_traits>
 #include <vector>
 
@@ -198,8 +200,10 @@ struct JacobiGeom {
   const double *ghi[3];
   int active[3];
   double coef;  // sum over active axes of 2 / dx^2
-  // reciprocals of dxsq and coef, rounded in the precision of the sweep
+  // reciprocals of dxsq and coef, rounded in the precision of the sweep, and
+  // the |x| from which on div_by() gives every quotient by them
   double rdxsq[3], rcoef;
+  double div_lo;
   // Curvilinear weights per vertex (NULL: Cartesian): the update is
   // (sum_a wsum[a] (prev + next) + wdiff[a] (next - prev) - lap) / wden.
   const double *wsum[3];
@@ -223,17 +227,38 @@ struct JacobiState {
 static_assert(sizeof(JacobiState) == PML_JACOBI_STATE_BYTES, "JacobiState layout");
 
 // x / d with r = 1 / d rounded to nearest: the product with r, two steps of
-// correction by the residual x - q d (exact in one fused multiply-add).  The
-// first brings q within one ulp, after which the second rounds correctly
-// (P. Markstein, "Computation of elementary functions on the IBM RISC
-// System/6000 processor", 1990), so the result is the quotient's for every
-// normal x / d; 5 operations where the compiler's division takes 11 and a
-// reciprocal.
+// correction by the residual x - q d.  The first brings q within one ulp,
+// after which the second rounds correctly (P. Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990), so the
+// result is the quotient's for |x| from div_least() on and for +0; a product
+// that overflows leaves NaN.  5 operations where the compiler's division takes
+// 11 and a reciprocal.
 template <typename T>
 __device__ __forceinline__ T div_by(T x, T d, T r) {
   T q = x * r;
   q = __builtin_elementwise_fma(__builtin_elementwise_fma(-d, q, x), r, q);
   return __builtin_elementwise_fma(__builtin_elementwise_fma(-d, q, x), r, q);
+}
+
+// The |x| from which on div_by() divides by each of the divisors as a division
+// does (or gives NaN), for a type of p bits and normal numbers from 2^emin on.
+// The last bit of a residual x - q d is at least 2^(e(x) - 2 p + 1), a
+// multiple of the least subnormal 2^(emin - p + 1) from e(x) = emin + p on,
+// and the quotient itself has to be normal.  Infinite where a divisor has no
+// normal reciprocal.
+template <typename T>
+static double div_least(const double *divisors, int n) {
+  constexpr int p = std::numeric_limits<T>::digits;
+  constexpr int emin = std::numeric_limits<T>::min_exponent - 1;
+  constexpr int emax = std::numeric_limits<T>::max_exponent - 1;
+  int least = emin + p;
+  for (int k = 0; k < n; ++k) {
+    const double d = static_cast<double>(static_cast<T>(divisors[k]));
+    if (!(d >= std::ldexp(1.0, emin + 2) && d <= std::ldexp(1.0, emax - 2)))
+      return std::numeric_limits<double>::infinity();
+    least = std::max(least, emin + 2 + std::ilogb(d));
+  }
+  return std::ldexp(1.0, least);
 }
 
 // The update of element t (field f of cell (idx)) from the iterate y.
@@ -275,12 +300,11 @@ __device__ __forceinline__ T jacobi_update(const T *y, I t, I f, I cell, const I
       acc = acc + static_cast<T>(g.wsum[a][cell]) * (prev + next);
       if (g.wdiff[a]) acc = acc + static_cast<T>(g.wdiff[a][cell]) * (next - prev);
     } else {
-      acc = acc + div_by(prev + next, static_cast<T>(g.dxsq[a]), static_cast<T>(g.rdxsq[a]));
+      acc = acc + (prev + next) / static_cast<T>(g.dxsq[a]);
     }
   }
   acc = acc - lap;
-  return g.wden ? acc / static_cast<T>(g.wden[cell])
-                : div_by(acc, static_cast<T>(g.coef), static_cast<T>(g.rcoef));
+  return acc / static_cast<T>(g.wden ? g.wden[cell] : g.coef);
 }
 
 // Each block writes its sum of squared updates to partials[blockIdx.x]
@@ -329,7 +353,9 @@ __global__ void k_jacobi(const T *y, T *yn, const T *lap, int64_t total, int nf,
 // its reduction and two barriers (1.2 us) below 20 x 20.
 // PLATE: one field on two axes, without vertex weights (grids of 3 x 3 and
 // more).  Vertices inside the grid read their neighbours without a branch
-// there; the general update is left to free vertices on an edge.
+// there and divide by div_by(); the general update is left to free vertices
+// on an edge.  A vertex with a numerator below div_least() or a result that is
+// not finite is divided as elsewhere, unless all three numerators are 0.
 template <typename T, int PER, bool PLATE>
 __global__ void __launch_bounds__(1024)
     k_jacobi_resident(T *y, const T *start, const T *__restrict__ lap, T scale, int total, int nf,
@@ -369,6 +395,7 @@ __global__ void __launch_bounds__(1024)
   const T dxsq0 = static_cast<T>(g.dxsq[0]), dxsq1 = static_cast<T>(g.dxsq[1]);
   const T rdxsq0 = static_cast<T>(g.rdxsq[0]), rdxsq1 = static_cast<T>(g.rdxsq[1]);
   const T coef = static_cast<T>(g.coef), rcoef = static_cast<T>(g.rcoef);
+  const T div_lo = static_cast<T>(g.div_lo);
   long long sweeps = 0;
   double norm = 0.0, sum = 0.0;
   bool done = false;
@@ -391,9 +418,16 @@ __global__ void __launch_bounds__(1024)
           const T left = L[max(t - 1, 0)], right = L[min(t + 1, total - 1)];
           idx[0] = quotient(t, m1);
           idx[1] = t - idx[0] * n1;
-          T acc = T(0) + div_by(up + down, dxsq0, rdxsq0);
-          acc = acc + div_by(left + right, dxsq1, rdxsq1);
-          nv[k] = div_by(acc - src[k], coef, rcoef);
+          const T a = up + down, b = left + right;
+          T acc = T(0) + div_by(a, dxsq0, rdxsq0);
+          acc = acc + div_by(b, dxsq1, rdxsq1);
+          const T c = acc - src[k];
+          nv[k] = div_by(c, coef, rcoef);
+          if (!(fmin(fmin(fabs(a), fabs(b)), fabs(c)) >= div_lo) ||
+              !(fabs(nv[k]) < static_cast<T>(INFINITY))) {
+            if (a != T(0) || b != T(0) || c != T(0))
+              nv[k] = (((T(0) + a / dxsq0) + b / dxsq1) - src[k]) / coef;
+          }
           if (idx[0] == 0 || idx[0] == n0 - 1 || idx[1] == 0 || idx[1] == n1 - 1)
             nv[k] = jacobi_update<T, int>(L, t, 0, t, idx, 1, g, src[k], nullptr);
         } else {
@@ -441,11 +475,12 @@ __global__ void __launch_bounds__(1024)
 // Whether the resident loop takes a grid, and its workgroup memory.  A sweep
 // of two launches takes 8 to 9 us whatever the size (of these), and 64 are
 // launched before the host looks.  Resident sweeps in FP64: plates between
-// constrained edges 1.2 us at 17 x 17, 2.7 at 64 x 64, 5.6 at 100 x 100, 8.0
-// at 129 x 129; with free edges (the general update in every wavefront) 2.3
-// at 45 x 45, 4.8 at 64 x 64, 9.4 at 100 x 100; other grids
-// 2.0 at 13^3, 5.4 at 17^3.  The lid-driven cavity on 65 x 65, 60 steps: 42 ms
-// with a host round trip and 128 launches a step, 1.6 ms in the device loop.
+// constrained edges 1.2 us at 17 x 17, 2.9 at 65 x 65, 6.1 at 100 x 100, 8.8
+// at 129 x 129 (7 to 9 % of it the test of the quotients' range); with free
+// edges (the general update in every wavefront) 6.8 at 65 x 65, 10.5 at
+// 90 x 90; other grids 4.3 at 13^3, 7.4 at 17^3.  The lid-driven cavity on
+// 65 x 65, 60 steps: 42 ms with a host round trip and 128 launches a step,
+// 1.6 ms in the device loop.
 constexpr int kResidentPer = 18;
 // Sweeps of one launch at most (some 100 ms on the largest grid): the host
 // looks at the loop's state in between.
@@ -817,6 +852,12 @@ static int jacobi_geom(int precision, const int64_t *shape, int n_fields, const 
   }
   g.rcoef = precision == PML_F32 ? static_cast<double>(1.0f / static_cast<float>(g.coef))
                                  : 1.0 / g.coef;
+  double divisors[4] = {g.coef};
+  int n_div = 1;
+  for (int a = 0; a < 3; ++a)
+    if (g.active[a]) divisors[n_div++] = g.dxsq[a];
+  g.div_lo = precision == PML_F32 ? div_least<float>(divisors, n_div)
+                                  : div_least<double>(divisors, n_div);
   g.stride[2] = n_fields;
   g.stride[1] = shape[2] * n_fields;
   g.stride[0] = shape[1] * shape[2] * n_fields;
