@@ -472,16 +472,19 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
-// Whether the resident loop takes a grid, and its workgroup memory.  A sweep
-// of two launches takes 8 to 9 us whatever the size (of these), and 64 are
-// launched before the host looks.  Resident sweeps in FP64: plates between
-// constrained edges 1.2 us at 17 x 17, 2.9 at 65 x 65, 6.1 at 100 x 100, 8.8
-// at 129 x 129 (7 to 9 % of it the test of the quotients' range); with free
-// edges (the general update in every wavefront) 6.8 at 65 x 65, 10.5 at
+// Which grids the resident loop takes.  A sweep of two launches takes 8.0 to
+// 8.5 us whatever the size (of these), and 64 are launched before the host
+// looks.  Resident sweeps in FP64: plates between constrained edges 1.2 us at
+// 17 x 17, 2.9 at 65 x 65, 6.1 at 100 x 100, 8.8 at 129 x 129 (7 to 9 % of it
+// the test of the quotients' range); with free edges 6.8 at 65 x 65, 10.5 at
 // 90 x 90; other grids 4.3 at 13^3, 7.4 at 17^3.  The lid-driven cavity on
 // 65 x 65, 60 steps: 42 ms with a host round trip and 128 launches a step,
 // 1.6 ms in the device loop.
 constexpr int kResidentPer = 18;
+// A sweep's time on two launches, and up to which the Poisson time loop stays
+// in one workgroup: its steps would each pay the host's look and the launches
+// beyond convergence (some 0.3 ms) outside.
+constexpr double kTwoLaunchUs = 8.4, kPoissonLoopUs = 10.0;
 // Sweeps of one launch at most (some 100 ms on the largest grid): the host
 // looks at the loop's state in between.
 constexpr int64_t kResidentSweeps = 16384;
@@ -492,11 +495,74 @@ static size_t resident_lds(int64_t total) {
 static bool is_plate(const JacobiGeom &g, int nf) {
   return nf == 1 && !g.wden && g.n[0] > 1 && g.n[1] > 1 && g.n[2] == 1;
 }
-static bool takes_resident(int precision, int64_t total, int nf, const JacobiGeom &g,
-                           bool constrained) {
-  const size_t lds = precision == PML_F64 ? resident_lds<double>(total) : resident_lds<float>(total);
-  const int64_t limit = !is_plate(g, nf) ? 5 * 1024 : (constrained ? kResidentPer * 1024 : 8 * 1024);
-  return total <= limit && lds <= 150 * 1024;
+
+// A plate's resident sweep by its runs of 64 vertices, a wavefront's step
+// each, of which `slow` hold a free vertex on an edge and run the general
+// update as well.  Run r is on SIMD r % 4, and the fullest SIMD counts: slow
+// is 4 times its share.  Measured against this, FP64 us: 129 x 129 all edges
+// fixed 8.8 / 8.7, none 16.0 / 16.0; 64 x 256 one column free 20.1 / 22.4;
+// 256 x 64 none fixed 22.7 / 22.4; FP32 129 x 129 6.8 / 6.7 and 12.6 / 13.1.
+static double resident_us(int precision, int64_t total, int64_t slow) {
+  const double runs = static_cast<double>((total + 63) / 64);
+  return precision == PML_F64 ? 1.1 + 0.0292 * runs + 0.054 * slow
+                              : 1.3 + 0.0208 * runs + 0.047 * slow;
+}
+
+// The slow runs of a plate with all its edges free.
+static int64_t edge_runs(int n0, int n1) {
+  int64_t on[4] = {0, 0, 0, 0};
+  const int total = n0 * n1;
+  for (int r = 0; 64 * r < total; ++r) {
+    const int a = 64 * r, b = std::min(a + 63, total - 1);
+    const bool inside = a / n1 == b / n1 && a >= n1 && b < total - n1 && a % n1 && (b + 1) % n1;
+    if (!inside) ++on[r % 4];
+  }
+  return 4 * *std::max_element(on, on + 4);
+}
+
+// The same of the plate's own constraints, into st->sweeps (one block of 1024).
+__global__ void __launch_bounds__(1024) k_edge_runs(const double *ycons, int n0, int n1,
+                                                    JacobiState *st) {
+  __shared__ int on[4];
+  if (threadIdx.x < 4) on[threadIdx.x] = 0;
+  __syncthreads();
+  const int total = n0 * n1;
+  for (int t0 = 0; t0 < total; t0 += 1024) {
+    const int t = t0 + threadIdx.x;
+    const int i = t / n1, j = t - i * n1;
+    const bool edge = t < total && (i == 0 || i == n0 - 1 || j == 0 || j == n1 - 1);
+    const bool slow = edge && ycons[t] != ycons[t];
+    if (__ballot(slow) && (threadIdx.x & 63) == 0) atomicAdd(&on[(t >> 6) & 3], 1);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) st->sweeps = 4 * max(max(on[0], on[1]), max(on[2], on[3]));
+}
+
+// Whether the resident loop takes a grid for at most `most_us` a sweep.  Where
+// that depends on which edge vertices are free, they are counted (one launch
+// and a look by the host, some 20 us).
+static int takes_resident(int precision, int64_t total, int nf, const JacobiGeom &g,
+                          const double *ycons, double most_us, JacobiState *js, hipStream_t st,
+                          bool *yes) {
+  *yes = false;
+  if (!is_plate(g, nf)) {
+    *yes = total <= 5 * 1024;
+    return PML_OK;
+  }
+  if (total > kResidentPer * 1024 || resident_us(precision, total, 0) > most_us) return PML_OK;
+  const int n0 = static_cast<int>(g.n[0]), n1 = static_cast<int>(g.n[1]);
+  int64_t slow = edge_runs(n0, n1);
+  if (ycons && resident_us(precision, total, slow) > most_us) {
+    hipLaunchKernelGGL(k_edge_runs, dim3(1), dim3(1024), 0, st, ycons, n0, n1, js);
+    PML_LAUNCH_CHECK();
+    long long counted = 0;
+    PML_HIP_CHECK(hipMemcpyAsync(&counted, &js->sweeps, sizeof(counted), hipMemcpyDeviceToHost,
+                                 st));
+    PML_HIP_CHECK(hipStreamSynchronize(st));
+    slow = counted;
+  }
+  *yes = resident_us(precision, total, slow) <= most_us;
+  return PML_OK;
 }
 
 template <typename T>
@@ -931,7 +997,12 @@ static int jacobi_solve(int precision, void *y, void *work, const void *lap,
   host.sweeps = 0;
   host.last_diff = 0.0;
   int64_t issued = 0;
-  if (takes_resident(precision, total, n_fields, g, ycons != nullptr)) {
+  bool resident = false;
+  if (int rc = takes_resident(precision, total, n_fields, g, ycons, kTwoLaunchUs, js, st,
+                              &resident);
+      rc != PML_OK)
+    return rc;
+  if (resident) {
     while (issued < max_sweeps) {
       const int64_t n = std::min<int64_t>(kResidentSweeps, max_sweeps - issued);
       hipLaunchKernelGGL(k_jacobi_init, dim3(1), dim3(64), 0, st, js);
@@ -1044,6 +1115,8 @@ extern "C" int pml_fdm_poisson_solve(int eq_id, const double *eq_params, int n_p
     return fail(PML_E_INVALID, "bad grid of a Poisson time loop");
   const int64_t fields = total_elems / plane;
   std::vector<JacobiGeom> geoms(n_poisson);
+  hipStream_t st = as_stream(stream);
+  auto *js = static_cast<JacobiState *>(jacobi_state);
   for (int k = 0; k < n_poisson; ++k) {
     if (field[k] < 0 || field[k] >= fields || source[k] < 0 || source[k] >= fields)
       return fail(PML_E_INVALID, "bad field of a Poisson equation");
@@ -1052,10 +1125,12 @@ extern "C" int pml_fdm_poisson_solve(int eq_id, const double *eq_params, int n_p
                              &total);
         rc != PML_OK)
       return rc;
-    if (!takes_resident(precision, plane, 1, geoms[k], ycons[k] != nullptr)) return PML_OK;
+    bool resident = false;
+    if (int rc = takes_resident(precision, plane, 1, geoms[k], ycons[k], kPoissonLoopUs, js, st,
+                                &resident);
+        rc != PML_OK || !resident)
+      return rc;
   }
-  hipStream_t st = as_stream(stream);
-  auto *js = static_cast<JacobiState *>(jacobi_state);
   const size_t esz = precision == PML_F64 ? 8 : 4;
   hipLaunchKernelGGL(k_jacobi_init, dim3(1), dim3(64), 0, st, js);
   PML_LAUNCH_CHECK();

@@ -886,7 +886,7 @@ class FDMOperator(Operator):
             if c is not None:
                 full = np.full(shape, np.nan)
                 full[c.mask] = c.values
-                c = torch.from_numpy(full.ravel()).to("cuda")
+                c = None if np.all(np.isnan(full)) else torch.from_numpy(full.ravel()).to("cuda")
             fixed.append(c)
         jacobi = torch.empty(nat.PML_JACOBI_STATE_BYTES // 8, dtype=torch.float64, device="cuda")
         sweeps = ctypes.c_int64(0)

@@ -662,7 +662,8 @@ class ThreePointCentralDifferenceMethod(NumericalDifferentiator):
             for f, c in enumerate(y_constraints):
                 if c is not None:
                     full[..., f : f + 1][..., c.mask] = c.values
-            ycons = torch.from_numpy(full.ravel()).to("cuda")
+            if not np.all(np.isnan(full)):
+                ycons = torch.from_numpy(full.ravel()).to("cuda")
         # ghost slabs per axis in "axis removed" layout
         glo, ghi, keep = [], [], []
         for axis in range(3):
