@@ -221,6 +221,13 @@ int pml_fdm_configs(int eq_id, int integrator_id, int precision);
 const char *pml_fdm_config_name(int eq_id, int integrator_id, int precision,
                                 int config);
 
+/* What PML_FLAG_AUTO does with a batch run by n_steps steps: plan[0 .. 3] =
+ * rows and columns of the output tiles, halo and steps a launch of the
+ * many-step kernel; all 0 where tile_config's variant runs it.  Reads the
+ * grids' vertex counts alone; needs no device. */
+int pml_fdm_auto_plan(int eq_id, int integrator_id, int precision, int ndim,
+                      const pml_grid *grids, int n_grids, int64_t n_steps, int *plan);
+
 /*
  * Standalone stencils on a (outer, n, inner) view of a contiguous array,
  * differentiating along the middle axis with spacing dx.  lo/hi are FP64

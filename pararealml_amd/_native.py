@@ -169,6 +169,9 @@ SIGNATURES = {
          POINTER(c_void_p), c_int, POINTER(c_int), POINTER(c_int), POINTER(c_void_p), c_void_p,
          c_double, c_double, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p],
     ),
+    "pml_fdm_auto_plan": (
+        c_int, [c_int, c_int, c_int, c_int, POINTER(PmlGrid), c_int, c_int64, POINTER(c_int)]
+    ),
     "pml_fdm_poisson_solve": (
         c_int,
         [c_int, POINTER(c_double), c_int, c_int, c_int, POINTER(PmlGrid), c_void_p, c_void_p,

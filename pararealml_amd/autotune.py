@@ -3,14 +3,17 @@
 For an (equation, integrator, precision, grid-size class) key it times every
 kernel variant ``libpml.so`` offers for that combination (tile height, fused
 steps per launch, workgroup size -- ``pml_fdm_configs`` /
-``pml_fdm_config_name``) on the live device, on a scratch batch of the
-caller's shape, and keeps the fastest.  Results persist as JSON in
+``pml_fdm_config_name``) and, where it has a plan for the batch, the many-step
+kernel on the live device, on a scratch batch of the caller's shape, and keeps
+the fastest.  Results persist as JSON in
 ``$PML_AUTOTUNE_CACHE`` (default ``~/.cache/pararealml_amd/autotune.json``)
 and are reused by ``FDMOperator`` when it is not given a ``tile_config``.
 The cache stores the variant's *name*; a lookup resolves it against the
 variants the loaded library offers, so an entry written by another build
 (pruned or reordered variants) falls back to the default variant instead
-of selecting a wrong or out-of-range one.
+of selecting a wrong or out-of-range one.  " > many-step" or " < many-step"
+after the name says that the many-step kernel was timed too and took less or
+more time than the variant; it stays off only in the second case.
 """
 
 import json
@@ -18,6 +21,8 @@ import os
 import threading
 from pathlib import Path
 from typing import Dict, List, Optional, Sequence
+
+MANY_STEP = "many-step"
 
 _lock = threading.Lock()
 _cache: Optional[Dict[str, str]] = None
@@ -76,58 +81,72 @@ def lookup(problem, integrator: int, precision: str, cells: Optional[int] = None
     if name is None:
         return 0
     if names is None:
-        from pararealml_amd import _device as dev
-        from pararealml_amd import _native as nat
-
-        names = variant_names(nat.PML_EQ[problem.eq_name], integrator,
-                              dev.precision_id(precision))
+        names = _offered(problem, integrator, precision)
     try:
-        return list(names).index(name)
+        return list(names).index(name.split(" ")[0])
     except ValueError:
         return 0
 
 
-def recorded(problem, integrator: int, precision: str, cells: Optional[int] = None) -> bool:
-    """Whether a tuning run recorded a variant for this key."""
+def _offered(problem, integrator: int, precision: str) -> List[str]:
+    from pararealml_amd import _device as dev
+    from pararealml_amd import _native as nat
+
+    return variant_names(nat.PML_EQ[problem.eq_name], integrator, dev.precision_id(precision))
+
+
+def many_step(problem, integrator: int, precision: str, cells: Optional[int] = None) -> bool:
+    """Whether batches of this key may run the many-step kernel: unless a
+    tuning run recorded a variant this library offers as the faster one."""
     with _lock:
-        return key_for(problem, integrator, precision, cells) in _load()
+        name = _load().get(key_for(problem, integrator, precision, cells), "")
+    variant, _, timed = name.partition(" ")
+    return timed != "< " + MANY_STEP or variant not in _offered(problem, integrator, precision)
 
 
 def tune(batch, d_t: float, n_steps: int = 64, repeats: int = 3, store: bool = True):
-    """Times every variant on ``batch`` (an ``FDMBatch``; its state is
-    advanced and therefore clobbered) and records the fastest.  Returns
-    ``(best_config, {config_name: seconds_per_step})``."""
+    """Times every variant and the many-step kernel on ``batch`` (an
+    ``FDMBatch``; its state is advanced and therefore clobbered) and records
+    the fastest.  Returns ``(best_config, {config_name: seconds_per_step})``:
+    the fastest variant, beside which ``"many-step"`` may be faster yet."""
+    import ctypes
+
     import torch
 
+    from pararealml_amd import _native as nat
+
     lib = batch.lib
-    n_cfg = lib.pml_fdm_configs(batch.eq_id, batch.integrator, batch.prec)
+    names = variant_names(batch.eq_id, batch.integrator, batch.prec)
+    plan = (ctypes.c_int * 4)()
+    nat.check(lib.pml_fdm_auto_plan(batch.eq_id, batch.integrator, batch.prec, batch.ndim,
+                                    batch.grids, len(batch.grid_problem), int(n_steps), plan))
+    candidates = [(name, dict(tile_config=cfg)) for cfg, name in enumerate(names)]
+    if plan[3]:
+        candidates.append((MANY_STEP, dict(auto=True)))
     timings = {}
-    best, best_t = 0, float("inf")
-    for cfg in range(n_cfg):
-        name = lib.pml_fdm_config_name(batch.eq_id, batch.integrator, batch.prec, cfg).decode()
-        batch.advance(d_t, 8, tile_config=cfg)  # warm-up
+    for name, choice in candidates:
+        batch.advance(d_t, 8, **choice)  # warm-up
         torch.cuda.synchronize()
         start = torch.cuda.Event(enable_timing=True)
         end = torch.cuda.Event(enable_timing=True)
         ts = []
         for _ in range(repeats):
             start.record(batch.stream)
-            batch.advance(d_t, n_steps, tile_config=cfg, use_graph=True)
+            batch.advance(d_t, n_steps, use_graph=True, **choice)
             end.record(batch.stream)
             end.synchronize()
             ts.append(start.elapsed_time(end) / 1e3 / n_steps)
-        t = min(ts)
-        timings[name] = t
-        if t < best_t:
-            best, best_t = cfg, t
+        timings[name] = min(ts)
+    best = min(range(len(names)), key=lambda cfg: timings[names[cfg]])
     if store:
         cells = sum(batch.problems[i].plane for i in batch.grid_problem)
         key = key_for(batch.problems[0], batch.integrator, batch.precision, cells)
-        best_name = lib.pml_fdm_config_name(batch.eq_id, batch.integrator, batch.prec,
-                                            best).decode()
+        entry = names[best]
+        if MANY_STEP in timings:
+            entry += (" > " if timings[MANY_STEP] < timings[entry] else " < ") + MANY_STEP
         with _lock:
             data = _load()
-            data[key] = best_name
+            data[key] = entry
             path = _cache_path()
             try:
                 path.parent.mkdir(parents=True, exist_ok=True)

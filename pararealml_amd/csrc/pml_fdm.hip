@@ -281,6 +281,19 @@ extern "C" const char *pml_fdm_config_name(int eq_id, int integrator_id, int pre
   return (*v)[config].name;
 }
 
+extern "C" int pml_fdm_auto_plan(int eq_id, int integrator_id, int precision, int ndim,
+                                 const pml_grid *grids, int n_grids, int64_t n_steps, int *plan) {
+  if ((ndim != 1 && ndim != 2) || !grids || n_grids <= 0 || n_steps < 0 || !plan)
+    return fail(PML_E_INVALID, "bad plan arguments");
+  const DeepPlan p =
+      deep_plan(find_deep(eq_id, integrator_id, precision, ndim), grids, n_grids, ndim, n_steps);
+  plan[0] = p.oy;
+  plan[1] = p.ox;
+  plan[2] = p.halo;
+  plan[3] = p.steps;
+  return PML_OK;
+}
+
 // The work-unit and grid tables of the allocation-free entry point live in
 // this file-scope device array (one copy per GPU, held for the life of the
 // process).  Host code never passes the array's name to a kernel: it uses

@@ -215,19 +215,21 @@ class FDMOperator(Operator):
 
     def kernel_choice(self, problem, n_grids: int = 1) -> dict:
         """``FDMBatch.advance`` arguments for a batch of ``n_grids`` grids of
-        ``problem``: ``tile_config_for``, and ``auto`` where neither the
-        constructor nor a tuning run chose that variant."""
-        from pararealml_amd.autotune import recorded
+        ``problem``: ``tile_config_for``, and ``auto`` (the many-step kernel
+        where it has a plan) unless the constructor was given that variant or
+        a tuning run found it faster."""
+        from pararealml_amd.autotune import many_step
 
-        chosen = self._tile_config is not None or recorded(
+        auto = self._tile_config is None and many_step(
             problem, dev.integrator_id(self._integrator), self._precision,
             cells=problem.plane * int(n_grids))
-        return dict(tile_config=self.tile_config_for(problem, n_grids), auto=not chosen)
+        return dict(tile_config=self.tile_config_for(problem, n_grids), auto=auto)
 
     def tune(self, cp, n_grids: int = 1, n_steps: int = 64, seed: int = 0) -> int:
-        """Times every kernel variant on a scratch batch of ``n_grids``
-        copies of ``cp``'s grid (random state, this operator's time step)
-        and records the fastest for the batch's size class; returns it."""
+        """Times every kernel variant, and the many-step kernel where it has a
+        plan, on a scratch batch of ``n_grids`` copies of ``cp``'s grid
+        (random state, this operator's time step) and records the fastest for
+        the batch's size class; returns the fastest variant."""
         import torch
 
         from pararealml_amd.autotune import tune
