@@ -474,7 +474,8 @@ class FDMOperator(Operator):
             static = (encode(cp.static_y_vertex_constraints),
                       no_dbc(cp.static_boundary_vertex_constraints[1]),
                       cp.static_y_vertex_constraints)
-        if family == "diffusion" and not dynamic and not implicit and mesh.dimensions <= 3:
+        if family == "diffusion" and not dynamic and not implicit \
+                and diff.takes_laplacian_solve(mesh.vertices_shape):
             # the right-hand side is one Laplacian: fused stages, no host work
             # between them
             y = torch.from_numpy(np.ascontiguousarray(
