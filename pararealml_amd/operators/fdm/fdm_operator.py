@@ -154,6 +154,17 @@ def ode_time_step(t0: float, n_steps: int, d_t: float) -> float:
     return ((t0 + n_steps * d_t) - t0) / n_steps
 
 
+def _built_in(differentiator, *names: str) -> bool:
+    """Whether these methods are the central difference method's own, which
+    the fused loops have built in."""
+    return all(
+        name not in vars(differentiator)
+        and getattr(type(differentiator), name)
+        is getattr(ThreePointCentralDifferenceMethod, name)
+        for name in names
+    )
+
+
 class FDMOperator(Operator):
     """A finite difference method based differential equation solver."""
 
@@ -475,7 +486,8 @@ class FDMOperator(Operator):
                       no_dbc(cp.static_boundary_vertex_constraints[1]),
                       cp.static_y_vertex_constraints)
         if family == "diffusion" and not dynamic and not implicit \
-                and diff.takes_laplacian_solve(mesh.vertices_shape):
+                and diff.takes_laplacian_solve(mesh.vertices_shape) \
+                and _built_in(diff, "laplacian", "_laplacian_terms"):
             # the right-hand side is one Laplacian: fused stages, no host work
             # between them
             y = torch.from_numpy(np.ascontiguousarray(
@@ -875,6 +887,8 @@ class FDMOperator(Operator):
 
         diff = self._differentiator
         if diff._max_sweeps < 16384:  # the limit is the caller's own
+            return False
+        if not _built_in(diff, "anti_laplacian"):
             return False
         shape = (problem.n0, problem.n1, 1)
         n = len(problem.y_laplacian)
