@@ -78,18 +78,20 @@ __device__ __forceinline__ T powi(T x, int k) {
 // back: s = sqrt(x) is off by r / (2 s), r = x - s^2, and the product by
 // pe, so x sqrt(x) = p + (pe + s r / 2).  Within 0.5005 ulp in FP64 on 400000
 // arguments in [0, 8] and 1e-100 .. 1e100 (pow: 1.28), and some 25 dependent
-// instructions where pow has hundreds.  Zero, infinity, negative values and NaN as pow.
+// instructions where pow has hundreds.  Zero, infinities, negative values and
+// NaN as pow (x sqrt(x) of -infinity is NaN, pow's limit there infinity).
 __device__ __forceinline__ double pow3h(double x) {
   const double s = sqrt(x);
   const double p = x * s;
   const double r = __builtin_fma(-s, s, x);
   const double pe = __builtin_fma(x, s, -p);
   const double v = p + __builtin_fma(0.5 * s, r, pe);
-  return fabs(p) < __builtin_inf() ? v : p;
+  if (fabs(p) < __builtin_inf()) return v;
+  return x == -__builtin_inf() ? -x : p;
 }
 __device__ __forceinline__ float pow3h(float x) {
   const double d = x;
-  return static_cast<float>(d * sqrt(d));
+  return x == -__builtin_inff() ? -x : static_cast<float>(d * sqrt(d));
 }
 
 // The operations on one or two values (every opcode that is neither a read
