@@ -163,7 +163,7 @@ def host_copy(a: np.ndarray) -> np.ndarray:
 
 
 def to_host(t) -> np.ndarray:
-    """A contiguous device tensor as a NumPy array in ordinary memory, after
+    """A device tensor as a contiguous NumPy array in ordinary memory, after
     the work queued on the current stream.  Most of torch's copy is the first
     touch of the destination's pages by one thread, which ``pml_download``
     shares out: 82 MB 19.5 ms / 2.9 ms, 20 MB 3.6 / 0.8, 4 MB 0.24 / 0.23;
@@ -172,7 +172,8 @@ def to_host(t) -> np.ndarray:
 
     nbytes = t.numel() * t.element_size()
     if nbytes < _THREADED_BYTES or t.dtype not in (torch.float64, torch.float32):
-        return t.cpu().numpy()
+        return t.cpu().contiguous().numpy()
+    t = t.contiguous()
     out = np.empty(tuple(t.shape), dtype=np.float64 if t.dtype == torch.float64 else np.float32)
     nat.check(nat.device_lib().pml_download(
         out.ctypes.data, t.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream))
@@ -189,6 +190,7 @@ def states_to_host(states, problem, spatial_shape) -> np.ndarray:
         if 8 * states.numel() < 1 << 20:  # sooner transposed here than launched there
             flat = states.cpu().numpy().reshape(n, problem.n_fields, problem.n0, problem.n1)
             return problem.from_device_layout(flat, spatial_shape)
+        states = states.contiguous()
         last = torch.empty_like(states)
         nat.check(nat.device_lib().pml_channel_last(
             states.data_ptr(), last.data_ptr(), problem.n_fields, problem.plane, n,
