@@ -162,6 +162,15 @@ def host_copy(a: np.ndarray) -> np.ndarray:
     return out
 
 
+def _download(t, out: np.ndarray) -> None:
+    """A contiguous device tensor into a contiguous array of the same type,
+    after the work queued on the current stream."""
+    import torch
+
+    nat.check(nat.device_lib().pml_download(
+        out.ctypes.data, t.data_ptr(), out.nbytes, torch.cuda.current_stream().cuda_stream))
+
+
 def to_host(t) -> np.ndarray:
     """A device tensor as a contiguous NumPy array in ordinary memory, after
     the work queued on the current stream.  Most of torch's copy is the first
@@ -173,11 +182,14 @@ def to_host(t) -> np.ndarray:
     nbytes = t.numel() * t.element_size()
     if nbytes < _THREADED_BYTES or t.dtype not in (torch.float64, torch.float32):
         return t.cpu().contiguous().numpy()
-    t = t.contiguous()
     out = np.empty(tuple(t.shape), dtype=np.float64 if t.dtype == torch.float64 else np.float32)
-    nat.check(nat.device_lib().pml_download(
-        out.ctypes.data, t.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream))
+    _download(t.contiguous(), out)
     return out
+
+
+# Device memory that transposed states take at most (one state, if that is
+# more): a trajectory may fill most of the card by itself.
+_TRANSPOSED_BYTES = 256 << 20
 
 
 def states_to_host(states, problem, spatial_shape) -> np.ndarray:
@@ -185,18 +197,25 @@ def states_to_host(states, problem, spatial_shape) -> np.ndarray:
     channel-last host array ``(n, *spatial_shape, fields)``."""
     import torch
 
-    n = states.shape[0]
-    if problem.n_fields > 1 and problem.plane > 1:
-        if 8 * states.numel() < 1 << 20:  # sooner transposed here than launched there
-            flat = states.cpu().numpy().reshape(n, problem.n_fields, problem.n0, problem.n1)
-            return problem.from_device_layout(flat, spatial_shape)
-        states = states.contiguous()
-        last = torch.empty_like(states)
+    n, elems = states.shape
+    shape = (n,) + tuple(spatial_shape) + (problem.n_fields,)
+    if problem.n_fields == 1 or problem.plane == 1:
+        return to_host(states).reshape(shape)
+    if 8 * states.numel() < 1 << 20:  # sooner transposed here than launched there
+        flat = states.cpu().numpy().reshape(n, problem.n_fields, problem.n0, problem.n1)
+        return problem.from_device_layout(flat, spatial_shape)
+    part = max(1, _TRANSPOSED_BYTES // (8 * elems))
+    last = torch.empty((min(part, n), elems), dtype=states.dtype, device=states.device)
+    out = np.empty((n, elems)) if n > part else None
+    for first in range(0, n, part):
+        some = states[first:first + part].contiguous()
         nat.check(nat.device_lib().pml_channel_last(
-            states.data_ptr(), last.data_ptr(), problem.n_fields, problem.plane, n,
+            some.data_ptr(), last.data_ptr(), problem.n_fields, problem.plane, len(some),
             torch.cuda.current_stream().cuda_stream))
-        states = last
-    return to_host(states).reshape((n,) + tuple(spatial_shape) + (problem.n_fields,))
+        if out is None:
+            return to_host(last).reshape(shape)
+        _download(last[:len(some)], out[first:first + len(some)])
+    return out.reshape(shape)
 
 
 _streams = {}

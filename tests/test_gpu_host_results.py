@@ -37,3 +37,24 @@ def test_strided_states_are_transposed_as_they_are():
     base = torch.rand(6000, 120, dtype=torch.float64, device="cuda")
     for states in (base.t(), base.t()[::2]):
         assert np.array_equal(dev.states_to_host(states, _Problem, (40, 50)), _want(states))
+
+
+@pytest.mark.parametrize("n", [1, 21, 22, 64])
+def test_transposed_states_need_bounded_device_memory(n, monkeypatch):
+    import torch
+
+    from pararealml_amd import _device as dev
+
+    print(f"case: bounded transposition {n}", flush=True)
+    limit = 1 << 20  # 21 states of 48 kB
+    monkeypatch.setattr(dev, "_TRANSPOSED_BYTES", limit, raising=False)
+    states = torch.rand(n + 21, 6000, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    got = dev.states_to_host(states, _Problem, (40, 50))
+    assert torch.cuda.max_memory_allocated() - before <= limit
+    assert np.array_equal(got, _want(states))
+    # one state beyond the limit goes by itself
+    monkeypatch.setattr(dev, "_TRANSPOSED_BYTES", 1, raising=False)
+    assert np.array_equal(dev.states_to_host(states, _Problem, (40, 50)), _want(states))
