@@ -154,6 +154,12 @@ def ode_time_step(t0: float, n_steps: int, d_t: float) -> float:
     return ((t0 + n_steps * d_t) - t0) / n_steps
 
 
+# Steps of one call of the Poisson time loop, as nearly as snapshots allow: the
+# host looks at its end (some 20 us, a step on the smallest grids) whether a
+# solve was cut short, and no more than these are taken again.
+_POISSON_STEPS = 256
+
+
 def _built_in(differentiator, *names: str) -> bool:
     """Whether these methods are the central difference method's own, which
     the fused loops have built in."""
@@ -875,10 +881,12 @@ class FDMOperator(Operator):
         return DeviceSolution(ivp, t[every::every], out, dev_y, vertex_oriented=True,
                               d_t=dt * every, copy=False)
 
-    def _poisson_loop(self, batch, problem, y_cons, d_cons, n_steps, traj, every) -> bool:
-        """The whole time loop on the device (``pml_fdm_poisson_solve``);
-        False where it does not cover the run, which then has to be stepped
-        from its initial state."""
+    def _poisson_loop(self, batch, problem, y_cons, d_cons, n_steps, traj, every) -> int:
+        """The time loop on the device (``pml_fdm_poisson_solve``), some
+        hundred steps a call; returns how many steps it took, after which the
+        batch holds their state (after none, nothing of use).  Fewer than
+        ``n_steps`` where it does not cover the grid or a solve needs more
+        sweeps than it takes."""
         import ctypes
 
         import torch
@@ -887,9 +895,9 @@ class FDMOperator(Operator):
 
         diff = self._differentiator
         if diff._max_sweeps < 16384:  # the limit is the caller's own
-            return False
+            return 0
         if not _built_in(diff, "anti_laplacian"):
-            return False
+            return 0
         shape = (problem.n0, problem.n1, 1)
         n = len(problem.y_laplacian)
         ghosts, fixed = ([], []), []
@@ -910,21 +918,36 @@ class FDMOperator(Operator):
         choice = self.kernel_choice(problem)
         pointers = lambda ts: (ctypes.c_void_p * len(ts))(  # noqa: E731
             *[None if a is None else a.data_ptr() for a in ts])
-        nat.check(batch.lib.pml_fdm_poisson_solve(
-            batch.eq_id, batch._params, len(batch.params), batch.integrator, batch.prec,
-            ctypes.byref(batch.grids[0]), batch.bc.data_ptr(), batch.hi.data_ptr(),
-            batch.work_hi.data_ptr(), batch.total, float(self._d_t), int(n_steps),
-            choice["tile_config"], nat.PML_FLAG_AUTO if choice["auto"] else 0, n,
-            (ctypes.c_int * n)(*[f for f, _, _ in problem.y_laplacian]),
-            (ctypes.c_int * n)(*[src for _, src, _ in problem.y_laplacian]),
-            (ctypes.c_double * n)(*[c for _, _, c in problem.y_laplacian]),
-            pointers(ghosts[0]), pointers(ghosts[1]), pointers(fixed), float(diff._tol),
-            traj.data_ptr(), int(every), jacobi.data_ptr(), ctypes.byref(sweeps),
-            batch._sptr()))
-        if not sweeps.value:
-            return False
-        diff.last_jacobi_sweeps = int(sweeps.value)
-        return True
+        done = 0
+        while done < n_steps:
+            # whole snapshot intervals, or a part of one
+            if every <= _POISSON_STEPS:
+                count = min(_POISSON_STEPS // every * every, n_steps - done)
+                snapshots = traj[done // every:].data_ptr()
+            else:
+                count = min(_POISSON_STEPS, every - done % every)
+                snapshots = None
+            start = batch.hi.clone() if done else None
+            nat.check(batch.lib.pml_fdm_poisson_solve(
+                batch.eq_id, batch._params, len(batch.params), batch.integrator, batch.prec,
+                ctypes.byref(batch.grids[0]), batch.bc.data_ptr(), batch.hi.data_ptr(),
+                batch.work_hi.data_ptr(), batch.total, float(self._d_t), int(count),
+                choice["tile_config"], nat.PML_FLAG_AUTO if choice["auto"] else 0, n,
+                (ctypes.c_int * n)(*[f for f, _, _ in problem.y_laplacian]),
+                (ctypes.c_int * n)(*[src for _, src, _ in problem.y_laplacian]),
+                (ctypes.c_double * n)(*[c for _, _, c in problem.y_laplacian]),
+                pointers(ghosts[0]), pointers(ghosts[1]), pointers(fixed), float(diff._tol),
+                snapshots, int(every), jacobi.data_ptr(), ctypes.byref(sweeps),
+                batch._sptr()))
+            if not sweeps.value:
+                if done:
+                    batch.hi.copy_(start)
+                return done
+            diff.last_jacobi_sweeps = int(sweeps.value)
+            done += count
+            if snapshots is None and done % every == 0:
+                batch.state_f64(traj[done // every - 1])
+        return done
 
     def _solve_with_poisson(self, ivp, problem, integ, t, n_steps, every, y0) -> Solution:
         """The time loop for equations with LHS.Y_LAPLACIAN components
@@ -959,10 +982,10 @@ class FDMOperator(Operator):
             traj = torch.empty((n_snap, problem.elems), dtype=torch.float64, device="cuda")
             tile = self.tile_config_for(problem)
             state = batch.hi  # field-major, the batch precision
-            fused = self._poisson_loop(batch, problem, y_cons, d_cons, n_steps, traj, every)
-            if not fused:  # a large grid, or a solve of many sweeps
+            first = self._poisson_loop(batch, problem, y_cons, d_cons, n_steps, traj, every)
+            if not first:  # a large grid, or a solve of many sweeps
                 batch.load_host([y0])
-            for i in range(0 if fused else n_steps):
+            for i in range(first, n_steps):
                 sources = {
                     f: (c * state[src * plane:(src + 1) * plane]).view(shape)
                     for f, src, c in problem.y_laplacian
