@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "pml_fdm_deep.h"
+#include "pml_launches.h"
 
 namespace pml {
 
@@ -485,21 +486,22 @@ static int fdm_solve_impl(int eq_id, const double *eq_params, int n_params,
       a.dt = dt;
       for (int i = 0; i < 6; ++i) a.p[i] = i < n_params ? eq_params[i] : 0.0;
       a.total = total_elems;
-      a.snap_every = static_cast<int>(
-          std::min<int64_t>(snapshots_hi ? snapshot_every : n_steps + 1, 1 << 30));
       a.n_tiles = tab.n_units;
       a.ndim = ndim;
       a.oy = plan.oy;
       a.ox = plan.ox;
       a.halo = plan.halo;
       for (int64_t done = 0; done < n_steps; done += a.steps) {
-        a.steps = static_cast<int>(std::min<int64_t>(plan.steps, n_steps - done));
+        const DeepLaunch l =
+            deep_launch(plan.steps, n_steps, done, snapshots_hi ? snapshot_every : 0);
+        a.steps = l.steps;
         a.in_hi = cur_hi;
         a.in_lo = cur_lo;
         a.out_hi = nxt_hi;
         a.out_lo = nxt_lo;
-        a.snap_idx = done / a.snap_every;
-        a.until = static_cast<int>(a.snap_every - done % a.snap_every);
+        a.snap_idx = l.snap_idx;
+        a.until = l.until;
+        a.snap_every = l.every;
         hipLaunchKernelGGL(fn, dim3(tab.n_units), dim3(threads), lds, st, a);
         PML_LAUNCH_CHECK();
         std::swap(cur_hi, nxt_hi);
