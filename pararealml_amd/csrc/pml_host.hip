@@ -175,6 +175,8 @@ extern "C" int pml_download(void *dst, const void *src, int64_t bytes, void *str
   hipStream_t st = as_stream(stream);
   int device = 0;
   PML_HIP_CHECK(hipGetDevice(&device));
+  // to the copying threads this name is another stream
+  if (st == hipStreamPerThread) PML_HIP_CHECK(hipStreamSynchronize(st));
   char *slots = take_staging();
   if (!slots) {  // no pinned memory to be had: the runtime's own copy
     PML_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
