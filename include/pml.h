@@ -504,14 +504,19 @@ int pml_prolong2x_cubic(int precision, const void *coarse, void *fine,
  *     once the derivative symbols have been computed into arrays.
  *   pml_ode_solve: advances `batch` independent states of an ODE system
  *     (n = n_outputs unknowns; input k is y[k]) by n_steps explicit steps
- *     (PML_INT_FE / MIDPOINT / RK4) of size dt, one thread per state, the
- *     whole time loop in one launch; y is (batch, n) in/out; the time of
+ *     (PML_INT_FE / MIDPOINT / RK4) of size dt, the whole time loop in one
+ *     launch: by the lanes of one wavefront per state where
+ *     pml_ode_wave_rounds gives the program a schedule for the batch, else
+ *     by one thread per state (the results are the same); y is (batch, n) in/out; the time of
  *     step s of state b is s * t_step[b] + t0[b] (the reference's
  *     linspace grid; t0, t_step device FP64 arrays); snapshots (may be
  *     NULL) receive every snapshot_every-th state at
  *     snapshots[(k * batch + b) * n].  Replaces FDMOperator.solve for
  *     systems without a mesh (fdm_operator.py:48-77 with
  *     numerical_integrator.py:42-132).
+ *   pml_ode_wave_rounds: rounds of the schedule by which pml_ode_solve runs
+ *     `batch` states of the program in the lanes of wavefronts; 0: by one
+ *     thread per state.
  */
 #define PML_EXPR_MAX_REGS 96
 #define PML_EXPR_MAX_IO 48
@@ -528,6 +533,7 @@ int pml_ode_solve(int precision, pml_program program, int integrator_id,
                   int64_t batch, const double *t0, const double *t_step,
                   double dt, int64_t n_steps, void *y, void *snapshots,
                   int64_t snapshot_every, void *stream);
+int pml_ode_wave_rounds(pml_program program, int64_t batch);
 
 /*
  * Solution post-processing on the device.  A snapshot stack holds n_t

@@ -94,6 +94,7 @@ SIGNATURES = {
         c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, POINTER(c_void_p)]
     ),
     "pml_program_destroy": (c_int, [c_void_p]),
+    "pml_ode_wave_rounds": (c_int, [c_void_p, c_int64]),
     "pml_expr_eval": (
         c_int,
         [c_int, c_void_p, POINTER(c_void_p), POINTER(c_int64), POINTER(c_void_p),

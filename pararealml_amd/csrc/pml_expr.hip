@@ -701,6 +701,13 @@ extern "C" int pml_expr_eval(int precision, pml_program p, const void *const *in
   return PML_OK;
 }
 
+extern "C" int pml_ode_wave_rounds(pml_program p, int64_t batch) {
+  if (!p) return 0;
+  const int64_t most =
+      p->n_instr * (p->elementary ? kWaveBatchPerInstrElementary : kWaveBatchPerInstr);
+  return batch <= most ? p->n_rounds : 0;
+}
+
 extern "C" int pml_ode_solve(int precision, pml_program p, int integrator_id, int64_t batch,
                              const double *t0, const double *t_step, double dt, int64_t n_steps,
                              void *y, void *snapshots, int64_t snapshot_every, void *stream) {
@@ -718,9 +725,7 @@ extern "C" int pml_ode_solve(int precision, pml_program p, int integrator_id, in
     return fail(PML_E_INVALID, "snapshot_every must be positive");
   if (n_steps == 0) return PML_OK;
   const size_t esz = precision == PML_F64 ? 8 : 4;
-  const int64_t max_wave_batch =
-      p->n_instr * (p->elementary ? kWaveBatchPerInstrElementary : kWaveBatchPerInstr);
-  if (p->n_rounds && batch <= max_wave_batch && (precision == PML_F64 || precision == PML_F32)) {
+  if (pml_ode_wave_rounds(p, batch) && (precision == PML_F64 || precision == PML_F32)) {
     const size_t lds = sizeof(WaveOp) * kWaveLanes * (p->n_rounds + 1) + esz * p->n_slots;
     hipStream_t st = as_stream(stream);
     auto launch = [&](auto kernel, auto *yp, auto *sp) {

@@ -5,10 +5,13 @@ both (down to 3 vertices an axis), on lines, on ragged batches, with snapshots
 every step, at intervals that do not divide a launch's steps and without,
 Dirichlet and Neumann edges mixed per side, the input constrained in the call."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
 import pararealml_amd as pml
+from pararealml_amd import _native as nat
 
 pytestmark = pytest.mark.gpu
 
@@ -40,7 +43,15 @@ def _problem(name, shape):
     return dev.device_problem(pml.ConstrainedProblem(eq, mesh, pairs[:len(shape)]))
 
 
-def _compare(name, shapes, integ, precision, steps, every):
+def _steps_a_launch(batch, steps):
+    """0: the streaming kernels run the batch."""
+    plan = (ctypes.c_int * 4)()
+    nat.check(batch.lib.pml_fdm_auto_plan(batch.eq_id, batch.integrator, batch.prec, batch.ndim,
+                                          batch.grids, len(batch.grid_problem), steps, plan))
+    return plan[3]
+
+
+def _compare(name, shapes, integ, precision, steps, every, taken=True):
     import torch
 
     from pararealml_amd import _device as dev
@@ -54,6 +65,7 @@ def _compare(name, shapes, integ, precision, steps, every):
     with torch.cuda.stream(stream):
         for auto in (False, True):
             b = dev.FDMBatch(problems, list(range(len(shapes))), precision, integ, stream)
+            assert (_steps_a_launch(b, steps) > 0) == taken
             b.load_host(ys)
             snaps = b.new_snapshots(steps // every) if every else None
             b.advance(D_T, steps, snaps, every, constrain_input=True, auto=auto)
@@ -93,7 +105,7 @@ def test_many_step_kernel_on_ragged_batches():
 
 
 def test_large_batches_keep_their_variant():
-    _compare("diffusion", [(700, 700)], 2, "float32", 3, 0)  # above 640 tiles
+    _compare("diffusion", [(700, 700)], 2, "float32", 3, 0, taken=False)  # above 640 tiles
 
 
 @pytest.mark.parametrize("precision", ["float64", "float32"])
@@ -101,7 +113,7 @@ def test_large_batches_keep_their_variant():
 @pytest.mark.parametrize("n", [4, 31, 65, 129])
 def test_navier_stokes_single_steps(n, integ, precision):
     """The step inside a Poisson time loop: algebraic fields, one step a
-    launch."""
+    launch; and several, which no rule on short runs keeps from the kernel."""
     import torch
 
     from pararealml_amd import _device as dev
@@ -117,7 +129,8 @@ def test_navier_stokes_single_steps(n, integ, precision):
         for auto in (False, True):
             b = dev.FDMBatch([problem], [0], precision, integ, stream, poisson_phase=True)
             b.load_host([y0])
-            for _ in range(3):
-                b.advance(D_T, 1, auto=auto)
+            assert _steps_a_launch(b, 3) > 0
+            for steps in (1, 1, 1, 3):
+                b.advance(D_T, steps, auto=auto)
             outs.append(b.state_f64().cpu().numpy())
     assert np.all(np.isfinite(outs[0])) and np.array_equal(*outs)

@@ -2,7 +2,8 @@
 of one wavefront per system, against the kernel of one thread per system
 (which a batch above the wavefront kernel's limit takes): the same operations,
 so the same bits, for systems with more than 64 independent instructions, with
-every kind of instruction, and with one variable.  The limit is 16384 systems."""
+every kind of instruction, and with one variable.  The limit is 256 systems per
+instruction of the program, 64 with elementary functions."""
 
 import ctypes
 
@@ -74,6 +75,7 @@ def test_wave_schedule_equals_the_serial_program(name, precision):
         # (the limit is at most 256 systems per instruction)
         for batch in (3, 256 * len(program.code) + 1):
             print(f"case: ode wave {name} {precision} {integ} batch {batch}", flush=True)
+            assert (lib.pml_ode_wave_rounds(program.handle(), batch) > 0) == (batch == 3)
             scale = 1.0 + 0.01 * torch.arange(batch, dtype=torch.float64).remainder(3)
             y = (torch.from_numpy(y0)[None] * scale[:, None]).to("cuda", dtype).contiguous()
             t0 = (0.25 * torch.arange(batch, dtype=torch.float64).remainder(3)).cuda()
