@@ -300,12 +300,15 @@ int pml_jacobi_sweep(int precision, const void *y_old, void *y_new,
  * 872-927): sweeps (as pml_jacobi_sweep, y -> work -> y ...) until
  * ||y_new - y_old||_2 <= tol, with the stopping test on the device (a sweep
  * after convergence does nothing) and the host reading the loop state once
- * per `batch` sweeps; a grid that fits one workgroup's memory runs the whole
- * loop in one launch (the host looks once per 16384 sweeps).  y holds the start (constraints already applied) and
- * receives the result; work is a second array of the same size; state is a
- * device buffer of PML_JACOBI_STATE_BYTES (8-byte aligned).  The update
- * norm is summed in a fixed order, so the sweep count and the result are
- * bitwise reproducible.  *sweeps_out = the
+ * per `batch` sweeps; small grids, where that is the faster place, run the
+ * whole loop in one workgroup (the host looks once per 16384 sweeps).  y
+ * holds the start (constraints already applied) and receives the result;
+ * work is a second array of the same size; state is a device buffer of
+ * PML_JACOBI_STATE_BYTES (8-byte aligned).  The update norm is summed in a
+ * fixed order, so the sweep count and the result are bitwise reproducible;
+ * the order in one workgroup is another one than by launches, so a loop whose
+ * norm ties with tol to the last bits can take a sweep more or less there.
+ * The iterates are the same.  *sweeps_out = the
  * sweeps taken, or -(sweeps issued) if max_sweeps ran out first; *diff_out
  * (may be NULL) = the last update norm.
  */
@@ -349,7 +352,8 @@ int pml_jacobi_solve_weighted(int precision, void *y, void *work, const void *la
  * per vertex, NaN where free; NULL: none).  y holds the start and receives
  * the end state; work holds 3 more states; snapshots (FP64) receives every
  * snapshot_every-th state.  The stages round as the separate stencil,
- * pml_weighted_add and pml_set_values calls do.  PML_F64 and PML_F32.
+ * pml_weighted_add and pml_set_values calls do.  At most 2^31 - 256
+ * vertices.  PML_F64 and PML_F32.
  */
 int pml_laplacian_solve(int precision, int integrator_id, const int64_t *shape,
                         const double *dx, const double *const *ghost_lo,
@@ -370,7 +374,7 @@ int pml_laplacian_solve(int precision, int integrator_id, const int64_t *shape,
  * holds the start and receives the end, work is a second state, snapshots
  * (FP64, NULL: none) receives every snapshot_every-th state, jacobi_state is
  * a device buffer of PML_JACOBI_STATE_BYTES.  *sweeps_out = the last solve's
- * sweeps, or 0 where the grid is too large for the device loop (nothing was
+ * sweeps, or 0 where the device loop does not take the grid (nothing was
  * done) or a solve needs more than 16384 sweeps (state and snapshots are then
  * unspecified) or there was no step: step with pml_fdm_solve and
  * pml_jacobi_solve instead.  flags: PML_FLAG_AUTO.  PML_F64 and PML_F32.

@@ -17,8 +17,9 @@ integrators and ``ThreePointCentralDifferenceMethod``.  Polar,
 cylindrical and spherical meshes, 3-D Cartesian ones, time-dependent
 boundary conditions and the implicit integrators run through a composed
 device loop (``_solve_composed``: the differentiator's device operators per
-stage) for the diffusion, convection-diffusion, wave, shallow-water,
-Burgers, Cahn-Hilliard and Navier-Stokes equations.
+stage; the diffusion equation with static conditions and an explicit
+integrator in ``pml_laplacian_solve``) for the diffusion, convection-diffusion,
+wave, shallow-water, Burgers, Cahn-Hilliard and Navier-Stokes equations.
 Anything else raises ``NotImplementedError``; there is no host fallback.
 
 Any other equation -- every ODE system and any user-defined
@@ -423,7 +424,10 @@ class FDMOperator(Operator):
         side the loop composes (diffusion, convection-diffusion, wave,
         shallow water, Burgers, Cahn-Hilliard with its LHS.Y potential,
         Navier-Stokes with its Poisson phase) in FP64 or FP32; other
-        equations raise ``NotImplementedError``.  Called directly, it also
+        equations raise ``NotImplementedError``.  The diffusion equation with
+        static conditions and an explicit integrator leaves the loop early:
+        ``pml_laplacian_solve`` fuses its stages (grids below 2^31 vertices,
+        the method's own Laplacian).  Called directly, it also
         runs Cartesian meshes (the tests compare it with the fused kernels)."""
         import torch
 
