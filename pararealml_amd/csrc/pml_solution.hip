@@ -148,9 +148,12 @@ __global__ __launch_bounds__(kInterpBlock) void k_interp(
 // of up to 128).  Lanes run along t, so every corner read is one contiguous
 // run of the point's snapshots; the results pass through LDS (dynamic,
 // ts x 33 values) and leave as rows of 32 consecutive points per snapshot.
-// The rows are written past the caches, which keep the stack for the corner
-// reads of scattered points: 65 snapshots of 257 x 257 at 400000 points
-// 151.0 -> 143.3 us (the reads, 832 MB, come at 6 TB/s).
+// The rows of one field are written past the caches, which keep the stack for
+// the corner reads of scattered points: 65 snapshots of 257 x 257 at 400000
+// points 151.0 -> 143.3 us (the reads, 832 MB, come at 6 TB/s).  Several
+// fields fill a line between them, and past the caches each would write its
+// part by itself: three fields of 65 snapshots of 65 x 65 at 400000 points in
+// order 464 us through the caches, 812 past them (two fields 244 / 358).
 constexpr int kTiPoints = 32;
 constexpr int kTiMaxSnaps = 128;
 
@@ -210,12 +213,15 @@ __global__ __launch_bounds__(kInterpBlock) void k_interp_ti(
       }
     }
     __syncthreads();
-    for (int e = tid; e < t_loc * kTiPoints; e += kInterpBlock) {
-      const int r = e / kTiPoints, q = e % kTiPoints;
-      if (q < n_loc)
-        __builtin_nontemporal_store(s_val[r * kRow + q],
-                                    &out[((t0 + r) * n_points + p0 + q) * C + c]);
-    }
+    // (two loops: one store under a condition loses the hint)
+    auto rows = [&](auto put) {
+      for (int e = tid; e < t_loc * kTiPoints; e += kInterpBlock) {
+        const int r = e / kTiPoints, q = e % kTiPoints;
+        if (q < n_loc) put(&out[((t0 + r) * n_points + p0 + q) * C + c], s_val[r * kRow + q]);
+      }
+    };
+    if (C == 1) rows([](T *to, T v) { __builtin_nontemporal_store(v, to); });
+    else rows([](T *to, T v) { *to = v; });
     __syncthreads();
   }
 }
