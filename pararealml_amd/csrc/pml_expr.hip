@@ -301,7 +301,38 @@ constexpr int kMaxWaveRounds = 95;   // 47.5 KiB of schedule
 // Van der Pol (10) 2048 6.9 / 14.1, 8192 25.2 / 14.1.  With elementary
 // functions (225 registers, 2 wavefronts per SIMD; 63 instructions) 4096 75 /
 // 93, 8192 146 / 93.
+// That holds for programs with several instructions a round.  The deeper a
+// program, the less this kernel shares out: its time for a batch beyond what
+// the chip holds at once is that of the batch's rounds, the serial kernel's
+// that of the instructions.  Both are estimated (WaveCost) from chains of 2 to
+// 40 operations, one and three side by side (FP64, us a right-hand side, at
+// once / serial, 50 RK4 steps): 40 square roots and additions (80 rounds), 256
+// systems 15 / 26, 1024 32 / 26, 21248 470 / 26; 16 instructions in 9 rounds,
+// 2048 systems 2.8 / 4.6, 4096 5.5 / 4.5.
 constexpr int64_t kWaveBatchPerInstr = 256, kWaveBatchPerInstrElementary = 64;
+
+// Microseconds a right-hand side: rounds_us is one system's alone, system_us
+// what each of many adds, serial_us the serial kernel's (up to 65536 systems).
+struct WaveCost {
+  double rounds_us = 0.4, system_us = 0.0, serial_us = 0.0;
+  int64_t at_once = 0;  // systems that the 256 CUs hold
+
+  void add_round(int kind) {
+    const bool fma = kind == WK_FMA;
+    const bool root = kind == OP_DIV || kind == OP_SQRT || kind == OP_POW3H;
+    rounds_us += fma ? 0.12 : (root ? 0.30 : 0.35);
+    system_us += fma ? 1.6e-4 : (root ? 2.6e-4 : 3.0e-4);
+  }
+  void add_instruction(int op) {
+    const bool plain = op <= OP_DIV || op == OP_NEG || op == OP_STORE || op == OP_SQRT ||
+                       op == OP_POW3H;
+    serial_us += plain ? 0.28 : (op == OP_POWI ? 0.60 : 0.33);
+  }
+  bool pays(int64_t batch) const {
+    const int64_t fills = (batch + at_once - 1) / at_once;
+    return (fills == 1 || fills * rounds_us <= serial_us) && batch * system_us <= serial_us;
+  }
+};
 
 // kAll false: programs of additions, products, divisions, square roots and
 // integer and three-halves powers only (the kernel without the elementary
@@ -420,7 +451,12 @@ struct pml_program_s {
   int *out_slots = nullptr;
   int n_rounds = 0, n_runs = 0, n_slots = 0;
   bool elementary = false;  // uses more than the short kernel's operations
+  WaveCost cost;
 };
+
+static size_t wave_lds(const pml_program_s *p, size_t value_bytes) {
+  return sizeof(WaveOp) * kWaveLanes * (p->n_rounds + 1) + value_bytes * p->n_slots;
+}
 
 // Schedules a validated program into rounds for k_ode_wave: slots in single
 // assignment, then, round by round, the instructions that share the branch
@@ -626,6 +662,12 @@ extern "C" int pml_program_create(const int32_t *code, int n_instr, const double
     for (const WaveRun &r : runs)
       p->elementary |= !(r.kind == WK_FMA || r.kind == OP_DIV || r.kind == OP_SQRT ||
                          r.kind == OP_POW3H);
+    for (const WaveRun &r : runs)
+      for (int k = 0; k < r.rounds; ++k) p->cost.add_round(r.kind);
+    for (int pc = 0; pc < n_instr; ++pc) p->cost.add_instruction(code[4 * pc]);
+    // by LDS, and by the registers: 8 wavefronts a SIMD, 2 with elementary functions
+    p->cost.at_once = 256 * std::min<int64_t>(p->elementary ? 8 : 32,
+                                              160 * 1024 / wave_lds(p, sizeof(double)));
   }
   if (e != hipSuccess) {
     if (p->code) (void)hipFree(p->code);
@@ -705,7 +747,7 @@ extern "C" int pml_ode_wave_rounds(pml_program p, int64_t batch) {
   if (!p) return 0;
   const int64_t most =
       p->n_instr * (p->elementary ? kWaveBatchPerInstrElementary : kWaveBatchPerInstr);
-  return batch <= most ? p->n_rounds : 0;
+  return p->n_rounds && batch <= most && p->cost.pays(batch) ? p->n_rounds : 0;
 }
 
 extern "C" int pml_ode_solve(int precision, pml_program p, int integrator_id, int64_t batch,
@@ -726,7 +768,7 @@ extern "C" int pml_ode_solve(int precision, pml_program p, int integrator_id, in
   if (n_steps == 0) return PML_OK;
   const size_t esz = precision == PML_F64 ? 8 : 4;
   if (pml_ode_wave_rounds(p, batch) && (precision == PML_F64 || precision == PML_F32)) {
-    const size_t lds = sizeof(WaveOp) * kWaveLanes * (p->n_rounds + 1) + esz * p->n_slots;
+    const size_t lds = wave_lds(p, esz);
     hipStream_t st = as_stream(stream);
     auto launch = [&](auto kernel, auto *yp, auto *sp) {
       hipLaunchKernelGGL(kernel, dim3(batch), dim3(kWaveLanes), lds, st, p->rounds, p->n_rounds,

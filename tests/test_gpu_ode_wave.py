@@ -3,7 +3,8 @@ of one wavefront per system, against the kernel of one thread per system
 (which a batch above the wavefront kernel's limit takes): the same operations,
 so the same bits, for systems with more than 64 independent instructions, with
 every kind of instruction, and with one variable.  The limit is 256 systems per
-instruction of the program, 64 with elementary functions."""
+instruction of the program, 64 with elementary functions, and lower where the
+instructions wait for one another."""
 
 import ctypes
 
@@ -117,3 +118,54 @@ def test_three_halves_power():
     # one FP64 rounding plus the compensated tail's second-order error
     assert np.max(np.abs(got[:-4] - ref) / ref) <= 0.52 * 2.0**-52
     assert got[-4] == 0.0 and np.isposinf(got[-3]) and np.isnan(got[-2]) and np.isnan(got[-1])
+
+
+def _nested(depth, width, f):
+    class Nested(DifferentialEquation):
+        def __init__(self):
+            super().__init__(0, width)
+
+        @property
+        def symbolic_equation_system(self):
+            out = []
+            for v in self.symbols.y:
+                for _ in range(depth):
+                    v = f(v)
+                out.append(v)
+            return SymbolicEquationSystem(out)
+
+    return Nested()
+
+
+@pytest.mark.parametrize("name,lanes,serial", [
+    # systems at once that run in lanes, and that run one a thread
+    ("roots-40", (1, 256), (1024, 5312, 21248)),
+    ("roots-10", (1, 256, 1024), (5888,)),
+    ("squares-40", (1, 1024), (5312, 21248)),
+    ("sines-40", (1, 256, 1024), (2688,)),
+    ("horner", (1, 1024, 2048), (4096,)),
+    ("lorenz", (1, 1024, 4608), (4609,)),
+    ("bodies-2", (1, 4096), (16384,)),
+])
+def test_deep_programs_share_out_less(name, lanes, serial):
+    import sympy as sp
+
+    from pararealml_amd import _native as nat
+    from pararealml_amd.operators.device_program import ode_program
+
+    print(f"case: ode route {name}", flush=True)
+    kind, _, depth = name.partition("-")
+    f = {"roots": lambda v: sp.sqrt(v + 2), "squares": lambda v: v**2 - sp.Rational(1, 3),
+         "sines": sp.sin}.get(kind)
+    if f is not None:
+        eq = _nested(int(depth), 1, f)
+    elif kind == "horner":
+        eq = _nested(1, 1, lambda y: ((((y / 2 + 1) * y - 2) * y + sp.Rational(3, 10)) * y
+                                      - sp.Rational(1, 10)) * y)
+    else:
+        eq = _system(name)[0]
+    program, lib = ode_program(eq), nat.device_lib()
+    for batch in lanes:
+        assert lib.pml_ode_wave_rounds(program.handle(), batch) > 0, batch
+    for batch in serial:
+        assert lib.pml_ode_wave_rounds(program.handle(), batch) == 0, batch
