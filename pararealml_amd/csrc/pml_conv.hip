@@ -5,8 +5,8 @@
 //    (v_mfma_f32_32x32x16_bf16).  Implicit GEMM: M = pixels, N = 64 output
 //    channels, K = 9 taps x 64 input channels.  A persistent workgroup of
 //    8 wavefronts keeps all 9 taps of the weights in LDS and loops over
-//    output tiles of 4 or 8 rows of 32 pixels; a pair of wavefronts computes
-//    one or two rows, 32 output channels each.  The same main loop serves the forward pass (epilogue: bias,
+//    output tiles of 4, 8 or 16 rows of 32 pixels; a pair of wavefronts
+//    computes one, two or four rows, 32 output channels each.  The same main loop serves the forward pass (epilogue: bias,
 //    GELU, BF16 pre-activation and activation) and the input gradient
 //    (weights pre-arranged flipped and transposed; epilogue: times GELU'
 //    of the previous layer's pre-activation).
@@ -53,7 +53,7 @@ __device__ __forceinline__ float gelu_grad_f(float z) {
 }
 
 // ---------------------------------------------------------------------------
-// conv64 (MFMA).  Output tile: 4 R = 4 or 8 rows x kTC = 32 columns x 64
+// conv64 (MFMA).  Output tile: 4 R = 4, 8 or 16 rows x kTC = 32 columns x 64
 // channels (the figures below for R = 2).  The input patch (10 x 34 pixels) sits in LDS as 144-byte rows
 // (64 BF16 channels + 16 bytes of padding: 16 lanes reading consecutive
 // rows hit all 64 banks once, and every patch address is a per-lane base
@@ -72,12 +72,12 @@ constexpr int kPC = kTC + 2;      // patch columns incl. halo
 constexpr int kPatchPitch = 144;  // bytes per patch pixel
 constexpr int kWBytes = 9 * 64 * 128;
 constexpr int kConvThreads = 512;
-// Rows per wavefront R: the tile has 4 R rows, R = 2 or 1 (conv_rows()).
+// Rows per wavefront R: the tile has 4 R rows, R = 1, 2 or 4 (conv_rows()).
 constexpr int conv_patch_rows(int R) { return 4 * R + 2; }
 constexpr size_t conv_lds(int R) {
   return static_cast<size_t>(conv_patch_rows(R)) * kPC * kPatchPitch + kWBytes;
 }
-static_assert(conv_lds(2) <= 160 * 1024, "conv64 LDS budget");
+static_assert(conv_lds(4) <= 160 * 1024, "conv64 LDS budget");
 
 // Byte offset of 16-byte chunk `chunk` (0..7) of weight row `row`.
 __device__ __forceinline__ int wswz(int row, int chunk) {
@@ -1087,19 +1087,34 @@ static int launch_conv64(const ConvArgs &a, hipStream_t st) {
   return PML_OK;
 }
 
-// Rows per wavefront of a launch: the fewer rounds of one workgroup per CU,
-// a round taking 4.4 us with one row and 8 us with two (beside some 3 us for
-// the launch and the weights).  Measured forward, one row / two (with four
-// rows, as tiles of 16, before): 1 x 33 x 33 7.1 / 9.6 (14.5), 1 x 129 x 129
-// 7.9 / 10.4 (15.5), 1 x 257 x 129 11.8 / 11.1 (16.1), 4 x 129 x 129 16.9 /
-// 18.9 (18.5), 8 x 129 x 129 25.5 / 25.5 (30.8), 16 x 129 x 129 41.7 / 41.3
-// (41.5) us; the input gradient of the last 38.4 / 38.0 (39.9).
-static int conv_rows(int images, int H, int tiles_w) {
-  auto us = [&](int r) {
-    const int64_t tiles = static_cast<int64_t>(images) * ((H + 4 * r - 1) / (4 * r)) * tiles_w;
-    return static_cast<double>((tiles + cu_count() - 1) / cu_count()) * (0.8 + 3.6 * r);
+// Rows per wavefront of a launch: of one and two the fewer rounds of one
+// workgroup per CU, a round taking 4.4 us with one row and 8 us with two
+// (beside some 3 us for the launch and the weights).  us with one / two / four
+// rows, forward: 1 x 33 x 33 7.4 / 9.9 / 14.8, 1 x 129 x 129 8.0 / 10.5 / 15.5,
+// 1 x 257 x 257 17.3 / 19.9 / 18.1, 8 x 129 x 129 25.7 / 25.9 / 30.8, 16 x 129
+// x 129 40.0 / 40.6 / 42.5, 32 x 129 x 129 69.2 / 66.9 / 70.4; the input
+// gradient of 16 x 129 x 129 37.9 / 38.4 / 40.7, of 64 x 128 x 128 114 / 107 /
+// 112.
+//
+// Forward launches of full tiles write two arrays without a pause, and how
+// well two rows do that depends on the card: four rows / two, on three cards,
+// 64 x 64 x 64 37.6 39.4 35.4 / 40.5 49.2 36.6, 32 x 64 x 64 22.1 22.8 23.0 /
+// 23.7 25.1 22.2, 16 x 128 x 128 37.4 39.7 36.1 / 39.4 47.5 36.0, 2 x 512 x 512
+// 71.4 70.9 64.6 / 68.6 82.5 62.2.  They take four rows, or one where its
+// rounds are fewer (12 x 128 x 128 34.6 / 31.6); above 7 rounds of four, two
+// rows are ahead on the mean (64 x 128 x 128 132 134 129 / 128 137 119).
+static int conv_rows(int mode, int images, int H, int W, int tiles_w) {
+  auto tiles = [&](int r) {
+    return static_cast<int64_t>(images) * ((H + 4 * r - 1) / (4 * r)) * tiles_w;
   };
-  return us(1) < us(2) ? 1 : 2;
+  auto rounds = [&](int r) {
+    return static_cast<double>((tiles(r) + cu_count() - 1) / cu_count());
+  };
+  const double pixels = static_cast<double>(images) * H * W;
+  const bool full = pixels >= 0.95 * 16 * kTC * tiles(4);
+  if (mode == kFwd && full && rounds(2) > 1.0 && rounds(4) < 8.0)
+    return 3.0 + 4.2 * rounds(1) < 3.9 + 15.7 * rounds(4) ? 1 : 4;
+  return 4.4 * rounds(1) < 8.0 * rounds(2) ? 1 : 2;
 }
 
 extern "C" int pml_conv64(int mode, const void *in, const void *wk, const float *bias,
@@ -1133,11 +1148,13 @@ extern "C" int pml_conv64(int mode, const void *in, const void *wk, const float 
     a.W = W;
     a.tiles_w = (W + kTC - 1) / kTC;
     a.bytes = static_cast<unsigned>(nb * img_bytes);
-    const int rows = conv_rows(nb, H, a.tiles_w);
+    const int rows = conv_rows(mode, nb, H, W, a.tiles_w);
     a.tiles_h = (H + 4 * rows - 1) / (4 * rows);
     a.n_tiles = nb * a.tiles_h * a.tiles_w;
     const int rc = mode == kFwd
-                       ? (rows == 2 ? launch_conv64<kFwd, 2>(a, st) : launch_conv64<kFwd, 1>(a, st))
+                       ? (rows == 4   ? launch_conv64<kFwd, 4>(a, st)
+                          : rows == 2 ? launch_conv64<kFwd, 2>(a, st)
+                                      : launch_conv64<kFwd, 1>(a, st))
                        : (rows == 2 ? launch_conv64<kBwd, 2>(a, st) : launch_conv64<kBwd, 1>(a, st));
     if (rc) return rc;
   }

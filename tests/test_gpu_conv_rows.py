@@ -1,6 +1,6 @@
-"""The 64 -> 64 convolution with tiles of 4 and of 8 rows (chosen by the number
-of tiles): images one row and column beside multiples of both tiles, and
-batches on either side of the choice, against a plain FP32 convolution of the
+"""The 64 -> 64 convolution with tiles of 4, of 8 and, forward, of 16 rows
+(chosen by the number of tiles): images one row and column beside multiples of
+the tiles, and batches on either side of the choice, against a plain FP32 convolution of the
 same BF16 operands on the CPU."""
 
 import ctypes
@@ -11,9 +11,11 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 # tiles of 4 rows x 32 columns: one; one and a remainder; 256 and 264 of them
-# (a round of the card's 256 CUs and one more), then several rounds
+# (a round of the card's 256 CUs and one more), then several rounds; 256
+# full tiles of 16 rows, forward in one round of them, and as many with a row
+# and two columns missing in each image
 SHAPES = [(1, 3, 5), (1, 4, 32), (1, 5, 33), (2, 9, 65), (1, 128, 256), (1, 132, 256),
-          (5, 129, 129)]
+          (5, 129, 129), (32, 64, 64), (32, 63, 62)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)
