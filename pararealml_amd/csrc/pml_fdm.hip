@@ -67,11 +67,11 @@ constexpr int64_t kDeepTiles = 640;
 //   FP64 Burgers, 500 on a line   6.6 / 5.7 -> 1.3   300 x 300 29.8 / 15.0 -> 8.2
 //   FP32 shallow water 513 x 385 29.8 / 16.6 -> 13.7 600 x 600 30.3 / 20.8 -> 18.8
 //   FP32 Cahn-Hilliard 300 x 300  6.5 / 2.2 -> 1.5   600 x 600 6.5 / 2.7 -> 2.8
-// Runs of one or two steps of fewer than four stages keep their variant: they
-// are a launch or two there, one and the copy back here (FE and midpoint on
-// 33 x 33 to 600 x 600 and batches, some 380 runs of each: one step 0.8 to 1.3
-// of the streaming time, two steps 0.4 to 1.4; RK4 0.2 to 1.1; three steps
-// 0.15 to 0.9).  A step whose result may stay where it is written (`leave`)
+// Runs of one or two steps of fewer than four stages, or on lines, keep their
+// variant: they are a launch or two there, one and the copy back here (FE and
+// midpoint on 33 x 33 to 600 x 600 and batches, some 380 runs of each: one step
+// 0.8 to 1.3 of the streaming time, two steps 0.4 to 1.4; RK4 0.2 to 1.1, on
+// lines 0.9 to 1.15 and 0.5 to 1.25; three steps 0.15 to 0.9).  A step whose result may stay where it is written (`leave`)
 // has no copy and gains the latency (the step of a lid-driven cavity's time
 // loop on 65 x 65: the 60-step run 1.80 -> 1.54 ms).
 // Regions above 1024 vertices hold two a thread, which three fields (and two
@@ -83,7 +83,7 @@ static DeepPlan deep_plan(const Deep &d, const pml_grid *grids, int n_grids, int
   DeepPlan best;
   double best_us = 0.0;
   int64_t values = 0;  // of one state
-  if (!d.fn[0] || n_steps < (leave || d.stages >= 4 ? 1 : 3)) return best;
+  if (!d.fn[0] || n_steps < (leave || (ndim == 2 && d.stages >= 4) ? 1 : 3)) return best;
   int64_t whole = 0;  // the largest grid's vertices
   int max0 = 1, max1 = 1;
   for (int g = 0; g < n_grids; ++g) {

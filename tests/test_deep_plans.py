@@ -1,7 +1,7 @@
-"""Runs of one and two steps: the many-step kernel takes those with four
-stages a step, whose passes it saves, and leaves the others, which are a
-launch or two of the streaming kernels, where they were; from three steps on
-it takes all (no GPU needed)."""
+"""Runs of one and two steps: the many-step kernel takes those on plates with
+four stages a step, whose passes it saves, and leaves the others, which are a
+launch or two of the streaming kernels, where they were; from three steps on it
+takes all (no GPU needed)."""
 
 import ctypes
 
@@ -34,6 +34,8 @@ def test_short_runs(eq, n, n_grids, prec):
 
 
 def test_short_runs_on_lines():
-    assert _steps("burgers", nat.PML_INT_FE, nat.PML_F64, 1, 500, 2) == 0
-    assert _steps("burgers", nat.PML_INT_RK4, nat.PML_F64, 1, 500, 1) == 1
-    assert _steps("burgers", nat.PML_INT_FE, nat.PML_F64, 1, 500, 3) == 3
+    for eq in ("burgers", "diffusion", "wave"):
+        for integ in (nat.PML_INT_FE, nat.PML_INT_RK4):
+            for n_steps in (1, 2):
+                assert _steps(eq, integ, nat.PML_F64, 1, 500, n_steps) == 0
+            assert _steps(eq, integ, nat.PML_F64, 1, 500, 3) == 3
